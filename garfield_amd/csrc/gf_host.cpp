@@ -367,7 +367,7 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
     ix.gidx.upload(gidx);
     ix.lrow.upload(lrow);
     {
-        std::vector<float> at(size_t(N) * a);
+        std::vector<float> at(size_t(N) * a + gf::kAttrPad, 0.0f);
         for (uint32_t r = 0; r < N; ++r)
             for (uint32_t d = 0; d < a; ++d) at[size_t(r) * a + d] = h.attrs[size_t(gidx[r]) * a + d];
         ix.attrs.upload(at);

@@ -38,6 +38,7 @@ inline uint32_t trav_dual_lds_bytes(uint32_t Lpad, uint32_t hsize) {
     return Lpad * 8 + 2 * kXSlots * 8 + 128 * 4 + hsize * 4;
 }
 constexpr uint32_t kMaxAttr = 8;      // attributes per point supported
+constexpr uint32_t kAttrPad = 4;      // floats behind the attribute array: a row's attributes are read in 16-byte loads
 constexpr uint32_t kMaxE = 4;         // cross edges per (point, cell) supported
 constexpr uint32_t kSelTile = 1024;   // rows per selectivity tile
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
@@ -73,7 +74,7 @@ void quantise_i8(const float* x, uint64_t n, uint32_t D, float alpha, std::vecto
 struct TravArgs {
     const char* vec;          // N rows of rowbytes, cell-major
     uint32_t rowbytes, nch;
-    const float* attrs;       // N*a, cell-major
+    const float* attrs;       // N*a, cell-major, at least kAttrPad readable floats behind the last row
     const uint32_t* graph;    // N*R cell-local neighbour ids, cell-major rows
     const uint32_t* cross;    // cell-local ids: edge e of row r into cell c at r*xrow + c*xcell + e
     uint64_t xrow, xcell;     // resident index: P*E, E; a streamed batch ("T" layout): E, rows*E

@@ -323,9 +323,13 @@ __device__ __forceinline__ float row_reduce_ref(const QReg<4, LPR, CPL>& q, cons
 // Distance of one row's chunks raw[0..NCH) (this lane's part) to the query:
 // per-virtual-lane fma chains, the in-lane butterfly levels, then the
 // cross-lane levels; the row's distance ends in the group's first lane.
+// A chunk beyond the row's nch (the lane read another of the row's chunks
+// in its place) leaves the chain as it is: the chunk's terms are 0.
 template <int VT, int LPR, int CPL>
-__device__ __forceinline__ float row_reduce_gen(const QReg<VT, LPR, CPL>& q, const uint4 (&raw)[RowPlan<LPR, CPL>::NCH]) {
+__device__ __forceinline__ float row_reduce_gen(const QReg<VT, LPR, CPL>& q, const uint4 (&raw)[RowPlan<LPR, CPL>::NCH],
+                                                uint32_t nch) {
     using RP = RowPlan<LPR, CPL>;
+    const uint32_t l = lane_id() % RP::PL;
     float s[RP::V];
 #pragma unroll
     for (int j = 0; j < RP::V; ++j) {
@@ -334,6 +338,7 @@ __device__ __forceinline__ float row_reduce_gen(const QReg<VT, LPR, CPL>& q, con
         for (int m = 0; m < CPL; ++m) {
             float x[kEpc<VT>];
             decode_chunk<VT>(raw[j * CPL + m], x);
+            const float acc0 = acc;
 #pragma unroll
             for (int e = 0; e < kEpc<VT>; ++e) {
                 float d;
@@ -341,6 +346,7 @@ __device__ __forceinline__ float row_reduce_gen(const QReg<VT, LPR, CPL>& q, con
                 else d = q.v[j * CPL + m][e] - x[e];
                 acc = __builtin_fmaf(d, d, acc);
             }
+            acc = lane_chunk<LPR, CPL>(l, j * CPL + m) < nch ? acc : acc0;
         }
         s[j] = acc;
     }
@@ -363,54 +369,117 @@ __device__ __forceinline__ float row_reduce_gen(const QReg<VT, LPR, CPL>& q, con
 }
 
 template <int VT, int LPR, int CPL>
-__device__ __forceinline__ float row_reduce(const QReg<VT, LPR, CPL>& q, const uint4 (&raw)[RowPlan<LPR, CPL>::NCH]) {
-    if constexpr (VT == 4) return row_reduce_ref<LPR, CPL>(q, raw);
-    else return row_reduce_gen<VT, LPR, CPL>(q, raw);
+__device__ __forceinline__ float row_reduce(const QReg<VT, LPR, CPL>& q, const uint4 (&raw)[RowPlan<LPR, CPL>::NCH],
+                                            uint32_t nch) {
+    if constexpr (VT == 4) {
+        // binary16 zeros in place of the chunks beyond nch, as the query holds
+        using RP = RowPlan<LPR, CPL>;
+        const uint32_t l = lane_id() % RP::PL;
+        uint4 x[RP::NCH];
+#pragma unroll
+        for (int k = 0; k < RP::NCH; ++k) {
+            const bool in = lane_chunk<LPR, CPL>(l, k) < nch;
+            x[k] = make_uint4(in ? raw[k].x : 0u, in ? raw[k].y : 0u, in ? raw[k].z : 0u, in ? raw[k].w : 0u);
+        }
+        return row_reduce_ref<LPR, CPL>(q, x);
+    } else {
+        return row_reduce_gen<VT, LPR, CPL>(q, raw, nch);
+    }
 }
 
-// Distances of the n rows listed in S[0..n) (LDS).  Lane j with compact
-// index ci (< n) receives the distance of row S[ci] in `dist`.
+// Distances of the n rows (1 to 64) listed in S[0..n) (LDS).  Lane j with
+// compact index ci (< n) receives the distance of row S[ci] in `dist`.  S
+// then holds the distances.
+// A batch first reads its rows from S, then issues every load, then reduces;
+// nothing in it depends on a lane: a group beyond n repeats the last row and
+// a lane with no chunk of the row repeats its last chunk (both are lines the
+// batch reads anyway), so no load sits behind an exec-mask branch and the
+// whole batch waits for memory once.  The distances meet their lanes through
+// S, one LDS round trip per call instead of one shuffle per pass.  With the
+// 16-byte attribute loads below, against loads behind per-lane branches and
+// one shuffle per pass (250k x 128 index): fp32 traversal of 2500 queries at
+// L = 100 2.36 -> 2.12 ms, dual-channel on u8 rows at L = 600 (591 queries)
+// 12.8 -> 11.3 ms; gather brute force of 777 queries over 150k x 100 fp32
+// 4.38 -> 3.43 ms.
 template <int VT, int LPR, int CPL>
 __device__ __forceinline__ void eval_rows(const QReg<VT, LPR, CPL>& q, const char* vec, uint32_t rowbytes,
-                                          uint32_t nch, const uint32_t* S, uint32_t n, uint32_t ci,
+                                          uint32_t nch, uint32_t* S, uint32_t n, uint32_t ci,
                                           float& dist) {
     using RP = RowPlan<LPR, CPL>;
     const uint32_t g = lane_id() / RP::PL, l = lane_id() % RP::PL;
     const uint32_t npass = (n + RP::RPP - 1) / RP::RPP;
+    uint32_t coff[RP::NCH];
+#pragma unroll
+    for (int k = 0; k < RP::NCH; ++k) {
+        const uint32_t c = lane_chunk<LPR, CPL>(l, k);
+        coff[k] = (c < nch ? c : nch - 1u) * 16u;
+    }
     for (uint32_t k0 = 0; k0 < npass; k0 += RP::NB) {
+        uint32_t rows[RP::NB];
         uint4 raw[RP::NB][RP::NCH];
 #pragma unroll
         for (int b = 0; b < RP::NB; ++b) {
             const uint32_t i = (k0 + b) * RP::RPP + g;
-            const char* row = i < n ? vec + size_t(S[i]) * rowbytes : nullptr;
-#pragma unroll
-            for (int k = 0; k < RP::NCH; ++k) {
-                const uint32_t c = lane_chunk<LPR, CPL>(l, k);
-                raw[b][k] = make_uint4(0u, 0u, 0u, 0u);
-                if (row && c < nch) raw[b][k] = load16(row, c);
-            }
+            rows[b] = S[i < n ? i : n - 1u];
         }
 #pragma unroll
         for (int b = 0; b < RP::NB; ++b) {
             if (k0 + b >= npass) break;
-            const float v = row_reduce<VT, LPR, CPL>(q, raw[b]);
-            const float t = __shfl(v, int((ci % RP::RPP) * RP::PL), 64);
-            if (ci < n && ci / RP::RPP == k0 + b) dist = t;
+            const char* row = vec + size_t(rows[b]) * rowbytes;
+#pragma unroll
+            for (int k = 0; k < RP::NCH; ++k) raw[b][k] = *reinterpret_cast<const uint4*>(row + coff[k]);
+        }
+#pragma unroll
+        for (int b = 0; b < RP::NB; ++b) {
+            if (k0 + b >= npass) break;
+            const float v = row_reduce<VT, LPR, CPL>(q, raw[b], nch);
+            const uint32_t i = (k0 + b) * RP::RPP + g;
+            if (l == 0 && i < n) S[i] = __float_as_uint(v);
         }
     }
+    wave_sync();
+    if (ci < n) dist = __uint_as_float(S[ci]);
+    wave_sync();
 }
 
-__device__ __forceinline__ bool row_pass(const float* attrs, uint32_t a, uint32_t row,
-                                         const float (&lo)[kMaxAttr], const float (&hi)[kMaxAttr]) {
+// Attributes of one row, read as one or two 16-byte loads whatever a is
+// (4-byte aligned; the attribute array is padded by kAttrPad floats, so the
+// last rows' loads stay inside it).  A load per attribute behind a test of a
+// made the compiler wait for the first attribute before it issued anything
+// else, a memory round trip per expansion.
+struct __attribute__((packed, aligned(4))) Attr4 {
+    float v[4];
+};
+struct RowAttrs {
+    Attr4 p0, p1;
+};
+__device__ __forceinline__ RowAttrs load_attrs(const float* attrs, uint32_t a, uint32_t row) {
+    RowAttrs r;
+    const float* src = attrs + size_t(row) * a;
+    r.p0 = *reinterpret_cast<const Attr4*>(src);
+    if (a > 4u) r.p1 = *reinterpret_cast<const Attr4*>(src + 4);
+    return r;
+}
+__device__ __forceinline__ bool attrs_pass(const RowAttrs& r, uint32_t a, const float (&lo)[kMaxAttr],
+                                           const float (&hi)[kMaxAttr]) {
     bool ok = true;
 #pragma unroll
-    for (uint32_t d = 0; d < kMaxAttr; ++d) {
-        if (d < a) {
-            const float v = attrs[size_t(row) * a + d];
-            ok = ok && (v >= lo[d]) && (v <= hi[d]);
+    for (uint32_t d = 0; d < 4; ++d) {
+        const float v = r.p0.v[d];
+        ok = ok && ((v >= lo[d] && v <= hi[d]) || d >= a);
+    }
+    if (a > 4u) {
+#pragma unroll
+        for (uint32_t d = 4; d < kMaxAttr; ++d) {
+            const float v = r.p1.v[d - 4];
+            ok = ok && ((v >= lo[d] && v <= hi[d]) || d >= a);
         }
     }
     return ok;
+}
+__device__ __forceinline__ bool row_pass(const float* attrs, uint32_t a, uint32_t row,
+                                         const float (&lo)[kMaxAttr], const float (&hi)[kMaxAttr]) {
+    return attrs_pass(load_attrs(attrs, a, row), a, lo, hi);
 }
 
 // Evaluate candidate rows held one per lane (lanes with need=false keep dist
@@ -428,22 +497,12 @@ __device__ __forceinline__ uint32_t eval_lanes(const QReg<VT, LPR, CPL>& q, cons
     wave_sync();
     if (need) S[ci] = row;
     wave_sync();
-    float av[kMaxAttr];
-    if (pass && chk) {
-#pragma unroll
-        for (uint32_t d = 0; d < kMaxAttr; ++d)
-            if (d < p.a) av[d] = p.attrs[size_t(row) * p.a + d];
-    }
+    RowAttrs av;
+    if (pass) av = load_attrs(p.attrs, p.a, chk ? row : 0u);
     const uint32_t n = __popcll(m);
     dist = __int_as_float(0x7F800000);
     if (n) eval_rows<VT, LPR, CPL>(q, p.vec, p.rowbytes, p.nch, S, n, ci, dist);
-    if (pass) {
-        bool ok = chk;
-#pragma unroll
-        for (uint32_t d = 0; d < kMaxAttr; ++d)
-            if (d < p.a) ok = ok && (av[d] >= (*lo)[d]) && (av[d] <= (*hi)[d]);
-        *pass = ok;
-    }
+    if (pass) *pass = chk && attrs_pass(av, p.a, *lo, *hi);
     wave_sync();
     return n;
 }
@@ -1407,17 +1466,18 @@ __global__ void k_assemble_full(const uint32_t* graph, const uint32_t* cross, co
 // Exact distances of the rows S[0..nrows) to the query, merged into the
 // top-K (lane t < K: t-th best by (distance, row)).
 template <int VT, int LPR, int CPL>
-__device__ void bf_flush(const QReg<VT, LPR, CPL>& qv, const TravArgs& p, const uint32_t* S, uint32_t nrows,
+__device__ void bf_flush(const QReg<VT, LPR, CPL>& qv, const TravArgs& p, uint32_t* S, uint32_t nrows,
                          uint64_t& top, uint64_t* T) {
     const uint32_t lane = lane_id(), K = p.K;
     {
         for (uint32_t base = 0; base < nrows; base += 64u) {
             const uint32_t nb = nrows - base < 64u ? nrows - base : 64u;
             const bool mine = lane < nb;
+            const uint32_t row = mine ? S[base + lane] : 0u;
             float d = 0.0f;
             eval_rows<VT, LPR, CPL>(qv, p.vec, p.rowbytes, p.nch, S + base, nb,
                                      mine ? lane : 0xFFFFFFFFu, d);
-            const uint64_t c = mine ? make_cand(d, S[base + lane], true) : kCandSent;
+            const uint64_t c = mine ? make_cand(d, row, true) : kCandSent;
             const uint64_t thr = ckey(readlane64(top, K - 1));
             const bool surv = mine && ckey(c) < thr;
             const uint64_t sm = ballot(surv);
