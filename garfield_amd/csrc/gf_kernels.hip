@@ -104,6 +104,16 @@ __device__ __forceinline__ bool hash_insert(uint32_t* H, uint32_t hsize, uint32_
     }
     return false;
 }
+__device__ __forceinline__ bool hash_contains(const uint32_t* H, uint32_t hsize, uint32_t key) {
+    uint32_t h = hash_slot(key, hsize);
+    for (uint32_t i = 0; i < hsize; ++i) {
+        const uint32_t v = H[h];
+        if (v == key) return true;
+        if (v == kEmpty) return false;
+        h = hash_next(h, hsize);
+    }
+    return false;
+}
 __device__ __forceinline__ void hash_clear(uint32_t* H, uint32_t hsize) {
     uint4* h4 = reinterpret_cast<uint4*>(H);
     const uint4 e = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
@@ -887,26 +897,62 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
                 keys[e] = kEmpty;
                 if (cv && e < E) keys[e] = p.cross[size_t(crow(ac)) * p.xrow + size_t(nxt) * p.xcell + e];
             }
-            // Slots filled in order 0..127 (the reference fills them
-            // concurrently); slot i follows candidate i % 64 and takes its
-            // first cross edge not yet taken, else the first free local id.
             uint32_t tk0 = kEmpty, tk1 = kEmpty;
-            for (uint32_t i = 0; i < kXSlots; ++i) {
-                const uint32_t c = i & 63u;
-                if (!((cvm >> c) & 1u)) continue;
-                uint32_t found = kEmpty;
+            if (E <= 2u) {
+                // The reference gives each candidate two slots; a slot takes
+                // the candidate's first cross edge not yet taken, else the
+                // first free local id.  With at most two edges every edge
+                // target ends up taken whatever the order, so the slots hold
+                // the distinct targets plus the smallest other ids: one
+                // insertion per edge into the (cleared) visited set, then a
+                // scan of ids 64 at a time.  Slot by slot, with the free-id
+                // search of each slot starting at 0, a cell change cost 118k
+                // cycles (64 cells, L = 250: 3.5M of a query's 11.2M).
+                uint32_t nt = 0;
 #pragma unroll
-                for (uint32_t e = 0; e < kMaxE; ++e) {
-                    if (e < E && found == kEmpty) {
-                        const uint32_t k = readlane32(keys[e], c);
-                        if (ballot(tk0 == k || tk1 == k) == 0) found = k;
-                    }
+                for (uint32_t e = 0; e < 2; ++e) {
+                    const bool isnew = keys[e] != kEmpty && hash_insert(H, hsize, keys[e]);
+                    const uint64_t m = ballot(isnew);
+                    if (isnew) S[nt + lanes_below(m)] = keys[e];
+                    nt += __popcll(m);
                 }
-                for (uint32_t rp = 0; found == kEmpty && rp < szx; ++rp)
-                    if (ballot(tk0 == rp || tk1 == rp) == 0) found = rp;
-                if (found != kEmpty) {
-                    if (i < 64u) tk0 = lane == i ? found : tk0;
-                    else tk1 = lane == i - 64u ? found : tk1;
+                wave_sync();
+                const uint32_t want = 2u * __popcll(cvm);
+                for (uint32_t id0 = 0; nt < want && id0 < szx; id0 += 64u) {
+                    const uint32_t id = id0 + lane;
+                    const bool free = id < szx && !hash_contains(H, hsize, id);
+                    const uint64_t m = ballot(free);
+                    const uint32_t pos = nt + lanes_below(m);
+                    if (free && pos < want) S[pos] = id;
+                    nt += __popcll(m);
+                }
+                nt = nt < want ? nt : want;
+                wave_sync();
+                if (lane < nt) tk0 = S[lane];
+                if (64u + lane < nt) tk1 = S[64u + lane];
+                wave_sync();
+            } else {
+                // more edges than slots: which edges a candidate's slots take
+                // depends on the order, 0..127 (the reference fills them
+                // concurrently).  Ids below `rp` are all taken.
+                uint32_t rp = 0;
+                for (uint32_t i = 0; i < kXSlots; ++i) {
+                    const uint32_t c = i & 63u;
+                    if (!((cvm >> c) & 1u)) continue;
+                    uint32_t found = kEmpty;
+#pragma unroll
+                    for (uint32_t e = 0; e < kMaxE; ++e) {
+                        if (e < E && found == kEmpty) {
+                            const uint32_t k = readlane32(keys[e], c);
+                            if (ballot(tk0 == k || tk1 == k) == 0) found = k;
+                        }
+                    }
+                    for (; found == kEmpty && rp < szx; ++rp)
+                        if (ballot(tk0 == rp || tk1 == rp) == 0) found = rp;
+                    if (found != kEmpty) {
+                        if (i < 64u) tk0 = lane == i ? found : tk0;
+                        else tk1 = lane == i - 64u ? found : tk1;
+                    }
                 }
             }
             uint64_t w0 = kCandSent, w1 = kCandSent;
@@ -1012,17 +1058,6 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
 }
 
 // ------------------------------------------------------ dual-channel search
-__device__ __forceinline__ bool hash_contains(const uint32_t* H, uint32_t hsize, uint32_t key) {
-    uint32_t h = hash_slot(key, hsize);
-    for (uint32_t i = 0; i < hsize; ++i) {
-        const uint32_t v = H[h];
-        if (v == key) return true;
-        if (v == kEmpty) return false;
-        h = hash_next(h, hsize);
-    }
-    return false;
-}
-
 // Index of the first entry of A[start..L) that is unexplored and whose row
 // lies in [rlo, rhi) (L if none).  The sentinel carries the explored bit.
 __device__ __forceinline__ uint32_t first_unexplored_in(const uint64_t* A, uint32_t L, uint32_t start,
