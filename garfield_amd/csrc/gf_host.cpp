@@ -270,7 +270,10 @@ void map_cells(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix, s
         size[h.global_pid[i]]++;
     }
     ix.offset_h.assign(P + 1, 0);
-    for (uint32_t c = 0; c < P; ++c) ix.offset_h[c + 1] = ix.offset_h[c] + size[c];
+    for (uint32_t c = 0; c < P; ++c) {
+        ix.offset_h[c + 1] = ix.offset_h[c] + size[c];
+        ix.max_cell = std::max(ix.max_cell, size[c]);
+    }
     for (uint32_t i = 0; i < N; ++i) {
         const uint32_t c = h.global_pid[i];
         const uint32_t r = ix.offset_h[c] + fill[c];
@@ -1070,10 +1073,15 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     // Visited-set size for the keys live between two resets (the list, the
     // slots of four expansions and a cell's cross slots; the dual channel's
     // expansions fill 2R slots).
-    const uint32_t hsize = gf::visited_slots(L + gf::kXSlots + (channels == 2 ? 10 * R : 4 * R));
+    const uint32_t live = L + gf::kXSlots + (channels == 2 ? 10 * R : 4 * R);
+    const gf::VisitedSet vs = channels == 2 ? gf::VisitedSet{gf::visited_slots(live), 0u}
+                                            : gf::visited_set(ix->max_cell, live);
+    const uint32_t hsize = vs.words;
     const uint32_t Lpad = round_up(L, 2);
     const uint32_t lds = channels == 2 ? gf::trav_dual_lds_bytes(Lpad, hsize) : gf::trav_lds_bytes(Lpad, hsize, ix->P);
-    GF_REQUIRE(lds <= 64 * 1024, GF_E_UNSUPPORTED, "L too large for the LDS budget");
+    // the limit on L is the hash table's, whichever form of the set runs
+    GF_REQUIRE(std::max(lds, channels == 2 ? 0u : gf::trav_lds_bytes(Lpad, gf::visited_slots(live), ix->P)) <= 64 * 1024,
+               GF_E_UNSUPPORTED, "L too large for the LDS budget");
 
     // device scalars: tot[2] pairs, [3] fits, [4] items, [8..11] traversal /
     // brute-force / empty / full-graph counts, [12..13] traversal range,
@@ -1114,6 +1122,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     a.counters = b->counters.p;
     a.a = ix->a; a.P = ix->P; a.R = R; a.E = ix->E; a.L = L; a.K = K; a.rl = rl;
     a.hsize = hsize;
+    a.vbits = vs.bits;
     a.offl = gf::trav_offsets_in_lds(ix->P) ? 1u : 0u;
     a.Lpad = Lpad;
     // The full-graph route: its own visited-set size (L + FD list and B

@@ -18,7 +18,7 @@ constexpr uint32_t kXStep = 64;       // candidates feeding the slots (gpu_graph
 constexpr uint32_t kOffLds = 1024;    // cell offsets (P + 1) the traversal keeps in LDS
 
 // LDS bytes of the traversal kernel: candidate list, slot scratch, row list,
-// visited set of hsize keys, and the P + 1 cell offsets when they fit.
+// visited set of hsize words, and the P + 1 cell offsets when they fit.
 inline bool trav_offsets_in_lds(uint32_t P) { return P + 1 <= kOffLds; }
 // Visited-set slots for at most `live` keys between two clears: a load
 // factor of at most 0.6 (linear probing then needs about 3.6 probes for a new
@@ -28,6 +28,23 @@ inline uint32_t visited_slots(uint32_t live) {
     const uint32_t s = (live * 5u + 2u) / 3u;
     const uint32_t r = (s + 63u) / 64u * 64u;
     return r < 256u ? 256u : r;
+}
+// The cell-by-cell traversal's visited set: a bit per cell-local id when the
+// largest cell's bits take no more LDS than the hash table or kVisBitsMax
+// bytes, else the hash table.  words: its LDS words; bits: ids it covers (0:
+// hash table of `words` slots).  The line is where the bits still leave
+// room for 15 waves per CU at L = 100.  Measured, hash table against bits:
+// 12.5k-point cells (1.6 KB), 654 queries, L = 250, 5.34 -> 3.91 ms;
+// 62.5k-point cells (7.8 KB), 1329 queries, L = 700, 17.0 -> 10.5 ms, 10k
+// queries, L = 100 (memory bound), 5.31 -> 5.26 ms.
+constexpr uint32_t kVisBitsMax = 8192;
+struct VisitedSet {
+    uint32_t words, bits;
+};
+inline VisitedSet visited_set(uint32_t max_cell, uint32_t live) {
+    const uint32_t slots = visited_slots(live), words = (max_cell + 2047u) / 2048u * 64u;
+    if (words * 4u <= kVisBitsMax || words <= slots) return {words, words * 32u};
+    return {slots, 0u};
 }
 inline uint32_t trav_lds_bytes(uint32_t Lpad, uint32_t hsize, uint32_t P) {
     return Lpad * 8 + kXSlots * 8 + 128 * 4 + hsize * 4 + (trav_offsets_in_lds(P) ? (P + 1) * 4 : 0);
@@ -95,7 +112,8 @@ struct TravArgs {
     uint32_t* out_ids;        // Q*K
     float* out_dist;          // Q*K
     uint32_t* counters;       // Q*GF_NCOUNTERS
-    uint32_t a, P, R, E, L, K, rl, hsize, Lpad;   // hsize: visited-set slots (visited_slots)
+    uint32_t a, P, R, E, L, K, rl, hsize, Lpad;   // hsize: visited-set words (visited_set, visited_slots)
+    uint32_t vbits;           // k_traverse: ids of the visited set's bit form (0: hash table)
     uint32_t offl;            // 1: the launch's LDS holds the P + 1 cell offsets (trav_lds_bytes)
     // Full-graph route (queries with postfilter or more cells): the graph
     // over every point, FD rows per row (cell-major rows, kEmpty = no edge),

@@ -114,11 +114,57 @@ __device__ __forceinline__ bool hash_contains(const uint32_t* H, uint32_t hsize,
     }
     return false;
 }
-__device__ __forceinline__ void hash_clear(uint32_t* H, uint32_t hsize) {
+__device__ __forceinline__ void hash_clear(uint32_t* H, uint32_t hsize, uint32_t v = kEmpty) {
     uint4* h4 = reinterpret_cast<uint4*>(H);
-    const uint4 e = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    const uint4 e = make_uint4(v, v, v, v);
     for (uint32_t i = lane_id(); i < hsize / 4u; i += 64u) h4[i] = e;
     wave_sync();
+}
+
+// Inserts the keys of U entries per lane (those with todo set): each round
+// issues one probe of every entry still looking for its slot before it waits
+// for any, so the rounds are the longest probe sequence of the call and not
+// the sum of one per entry.
+template <uint32_t U>
+__device__ __forceinline__ void hash_insert_many(uint32_t* H, uint32_t hsize, const uint32_t (&key)[U], bool (&todo)[U]) {
+    uint32_t h[U], old[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) h[u] = hash_slot(key[u], hsize);
+    for (uint32_t i = 0; i < hsize; ++i) {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) old[u] = todo[u] ? atomicCAS(&H[h[u]], kEmpty, key[u]) : kEmpty;
+        bool any = false;
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            todo[u] = todo[u] && old[u] != kEmpty && old[u] != key[u];
+            h[u] = hash_next(h[u], hsize);
+            any |= todo[u];
+        }
+        if (!ballot(any)) break;
+    }
+}
+
+// Visited set of the cell-by-cell traversal, whose keys are cell-local ids:
+// one bit per id (vbits of them, no fewer than the largest cell holds) where
+// visited_set chose that, else the hash table (vbits 0).  An insertion is
+// then one LDS atomic instead of a probe sequence, and a rebuild waits for
+// none of its insertions.
+__device__ __forceinline__ bool vis_insert(uint32_t* H, uint32_t hsize, uint32_t vbits, uint32_t key) {
+    if (vbits) {
+        // an id beyond the bits (the first cell's entries are put in by point
+        // id, as the reference does) is no cell's local id: nothing asks for it
+        if (key >= vbits) return true;
+        const uint32_t bit = 1u << (key & 31u);
+        return (atomicOr(&H[key >> 5], bit) & bit) == 0;
+    }
+    return hash_insert(H, hsize, key);
+}
+__device__ __forceinline__ void vis_clear(uint32_t* H, uint32_t hsize, uint32_t vbits) {
+    hash_clear(H, hsize, vbits ? 0u : kEmpty);
+}
+__device__ __forceinline__ bool vis_contains(const uint32_t* H, uint32_t hsize, uint32_t vbits, uint32_t key) {
+    if (vbits) return (H[key >> 5] >> (key & 31u)) & 1u;
+    return hash_contains(H, hsize, key);
 }
 
 // ----------------------------------------------------------- row distances
@@ -658,44 +704,50 @@ __device__ __forceinline__ uint32_t first_unexplored(const uint64_t* A, uint32_t
     return L;
 }
 
-// Cell offsets for the visited-set keys of other cells' rows: with at most
-// 16 cells, offset[0..15] in (wave-uniform) registers; with up to kOffLds - 1
-// cells, an LDS copy O of offset[0..P]; beyond, none (lrow[] is gathered).
-struct CellOffs {
-    const uint32_t* O;
-    uint32_t P;
-    uint32_t o[16];
-};
-
-__device__ __forceinline__ void cell_offs_init(CellOffs& co, const TravArgs& p, uint32_t* O) {
-    co.O = O;
-    co.P = p.P;
+// Cell-local ids of U rows per lane, for the visited set: arithmetic inside
+// the cell [off, offn); for rows of other cells, row - offset[c] for the cell
+// c holding it (rows are cell-major, so this is lrow[row]), c found by a
+// binary search of the offsets' LDS copy O, the U searches in step so that a
+// round waits for LDS once.  Without the copy (too many cells) lrow[] is
+// gathered.  nlrow counts the rows of other cells.
+template <uint32_t U>
+__device__ __forceinline__ void local_keys(const TravArgs& p, const uint32_t* O, const uint32_t (&row)[U],
+                                           const bool (&in)[U], uint32_t off, uint32_t offn, uint32_t (&key)[U],
+                                           uint32_t& nlrow) {
+    if (O) {
+        uint32_t c[U], base[U];
 #pragma unroll
-    for (uint32_t t = 0; t < 16; ++t) co.o[t] = t <= p.P ? p.offset[t] : 0u;
-}
-
-// Cell-local key of a candidate row for the visited set: arithmetic inside
-// the cell [off, offn); for rows of other cells, row - offset[c] for the
-// cell c holding it (rows are cell-major, so this is lrow[row]).
-__device__ __forceinline__ uint32_t local_key(const TravArgs& p, const CellOffs& co, uint32_t row, uint32_t off,
-                                              uint32_t offn, uint32_t& nlrow) {
-    if (row >= off && row < offn) return row - off;
-    ++nlrow;
-    if (co.P <= 16) {
-        // the largest offset <= row (offsets ascend; empty cells repeat one)
-        uint32_t base = 0;
+        for (uint32_t u = 0; u < U; ++u) {
+            c[u] = 0;
+            base[u] = 0;
+        }
+        // the largest c with O[c] <= row (offsets ascend, O[0] = 0; empty cells repeat one)
+        for (uint32_t step = p.P > 1u ? 1u << (31 - __builtin_clz(p.P - 1u)) : 0u; step; step >>= 1) {
+            uint32_t o[U];
 #pragma unroll
-        for (uint32_t t = 1; t < 16; ++t)
-            if (t < co.P && row >= co.o[t]) base = co.o[t];
-        return row - base;
+            for (uint32_t u = 0; u < U; ++u) o[u] = O[c[u] + step < p.P ? c[u] + step : p.P];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const bool up = o[u] <= row[u];
+                base[u] = up ? o[u] : base[u];
+                c[u] = up ? c[u] + step : c[u];
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const bool here = row[u] >= off && row[u] < offn;
+            nlrow += in[u] && !here;
+            key[u] = row[u] - (here ? off : base[u]);
+        }
+    } else {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const bool here = row[u] >= off && row[u] < offn;
+            nlrow += in[u] && !here;
+            key[u] = row[u] - off;
+            if (in[u] && !here) key[u] = p.lrow[row[u]];
+        }
     }
-    if (!co.O) return p.lrow[row];
-    uint32_t lo = 0, hi = co.P;   // O[lo] <= row < O[hi]
-    while (hi - lo > 1u) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (co.O[mid] <= row) lo = mid; else hi = mid;
-    }
-    return row - co.O[lo];
 }
 
 // Insert the rows of the valid entries of A[0..L), four per lane at a time,
@@ -728,34 +780,33 @@ __device__ void hash_add_rows(uint32_t* H, uint32_t hsize, const uint64_t* A, ui
     wave_sync();
 }
 
-// Insert the keys of A[0..L), four per lane at a time: their keys are
-// computed, then their first probes issued, before any probe's result is
-// awaited (a set: the insertion order does not change membership).
-__device__ void hash_add_list(const TravArgs& p, const CellOffs& co, uint32_t* H, const uint64_t* A, uint32_t L,
-                              uint32_t off, uint32_t offn, uint32_t& nlrow) {
+// Insert the cell-local keys of A[0..L) and of one more candidate per lane
+// into the visited set, U list entries per lane at a time (a set: the order
+// of the insertions does not change membership).
+__device__ void vis_add_list(const TravArgs& p, const uint32_t* O, uint32_t* H, const uint64_t* A, uint32_t L,
+                             uint64_t more, uint32_t off, uint32_t offn, uint32_t& nlrow) {
     constexpr uint32_t U = 4;
-    const uint32_t hsize = p.hsize;
+    const uint32_t hsize = p.hsize, vbits = p.vbits;
+    // the lane's further candidate rides in the last batch of the list
     for (uint32_t base = 0; base < L; base += 64u * U) {
-        uint32_t key[U], h[U], old[U];
-        bool todo[U];
+        uint32_t row[U + 1], key[U + 1];
+        bool todo[U + 1];
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
+        for (uint32_t u = 0; u < U + 1; ++u) {
             const uint32_t i = base + u * 64u + lane_id();
-            const uint64_t c = i < L ? A[i] : kCandSent;
+            uint64_t c = kCandSent;
+            if (u < U) c = i < L ? A[i] : kCandSent;
+            else if (base + 64u * U >= L) c = more;
             todo[u] = cvalid(c);
-            key[u] = todo[u] ? local_key(p, co, crow(c), off, offn, nlrow) : 0u;
-            h[u] = hash_slot(key[u], hsize);
+            row[u] = todo[u] ? crow(c) : off;
         }
+        local_keys<U + 1>(p, O, row, todo, off, offn, key, nlrow);
+        if (vbits) {
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) old[u] = todo[u] ? atomicCAS(&H[h[u]], kEmpty, key[u]) : kEmpty;
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-            if (!todo[u] || old[u] == kEmpty || old[u] == key[u]) continue;
-            for (uint32_t j = 0; j + 1u < hsize; ++j) {
-                h[u] = hash_next(h[u], hsize);
-                const uint32_t o2 = atomicCAS(&H[h[u]], kEmpty, key[u]);
-                if (o2 == kEmpty || o2 == key[u]) break;
-            }
+            for (uint32_t u = 0; u < U + 1; ++u)
+                if (todo[u]) atomicOr(&H[key[u] >> 5], 1u << (key[u] & 31u));
+        } else {
+            hash_insert_many<U + 1>(H, hsize, key, todo);
         }
     }
     wave_sync();
@@ -794,12 +845,11 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
     const uint32_t q = p.sched[si];
     const uint32_t hsize = p.hsize;
     const uint32_t L = p.L, R = p.R, P = p.P, E = p.E;
+    const uint32_t vbits = p.vbits;
     // cell offsets for the visited-set keys of other cells' rows
     uint32_t* O = p.offl ? H + hsize : nullptr;
     if (O)
         for (uint32_t i = lane; i <= P; i += 64u) O[i] = p.offset[i];
-    CellOffs co;
-    cell_offs_init(co, p, O);
 
     QReg<VT, LPR, CPL> qv;
     load_query<VT, LPR, CPL>(qv, p.queries + size_t(q) * p.qbytes, p.nch);
@@ -810,7 +860,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
         hi[d] = d < p.a ? p.hi[size_t(q) * p.a + d] : 0.0f;
     }
     for (uint32_t i = lane; i < L; i += 64u) A[i] = kCandSent;
-    hash_clear(H, hsize);   // ends with a wave_sync
+    vis_clear(H, hsize, vbits);   // ends with a wave_sync
     uint32_t n_expand = 0, n_dist = 0, n_attr = 0, n_cross = 0, n_lrow = 0;
     uint64_t rc = kCandSent, bleft = kCandSent;
 
@@ -828,7 +878,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
         bool pass = false;
         if (mine) {
             row = off0 + p.entry[lane] % sz0;
-            hash_insert(H, p.hsize, p.gidx[row]);
+            vis_insert(H, hsize, vbits, p.gidx[row]);
             pass = row_pass(p.attrs, p.a, row, lo, hi);
         }
         wave_sync();
@@ -846,11 +896,8 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
 
         for (uint32_t it = 0; it < kMaxIter; ++it) {
             if ((it + 1) % kHashReset == 0) {          // gpu_graph.cu:3441-3454
-                hash_clear(H, hsize);
-                hash_add_list(p, co, H, A, L, off, offn, n_lrow);
-                if (lane < R && cvalid(bleft))
-                    hash_insert(H, p.hsize, local_key(p, co, crow(bleft), off, offn, n_lrow));
-                wave_sync();
+                vis_clear(H, hsize, vbits);
+                vis_add_list(p, O, H, A, L, lane < R ? bleft : kCandSent, off, offn, n_lrow);
             }
             const uint32_t sel = first_unexplored(A, L, scan);
             if (sel == L) break;
@@ -868,7 +915,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
             if (mine) {
                 const uint32_t nl = p.graph[size_t(srow) * R + lane];
                 nrow = off + nl;
-                isnew = hash_insert(H, p.hsize, nl);
+                isnew = vis_insert(H, hsize, vbits, nl);
             }
             n_attr += R;
             float d;
@@ -882,7 +929,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
         // End of cell (gpu_graph.cu:3555-3560).
         for (uint32_t i = lane; i < L; i += 64u) A[i] = A[i] | 2u;
         wave_sync();
-        hash_clear(H, hsize);
+        vis_clear(H, hsize, vbits);
         if (pi + 1 < cnt) {                             // gpu_graph.cu:3564-3642
             const uint32_t nxt = cl[pi + 1];
             const uint32_t offx = p.offset[nxt], offxn = p.offset[nxt + 1], szx = offxn - offx;
@@ -911,7 +958,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
                 uint32_t nt = 0;
 #pragma unroll
                 for (uint32_t e = 0; e < 2; ++e) {
-                    const bool isnew = keys[e] != kEmpty && hash_insert(H, hsize, keys[e]);
+                    const bool isnew = keys[e] != kEmpty && vis_insert(H, hsize, vbits, keys[e]);
                     const uint64_t m = ballot(isnew);
                     if (isnew) S[nt + lanes_below(m)] = keys[e];
                     nt += __popcll(m);
@@ -920,7 +967,7 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
                 const uint32_t want = 2u * __popcll(cvm);
                 for (uint32_t id0 = 0; nt < want && id0 < szx; id0 += 64u) {
                     const uint32_t id = id0 + lane;
-                    const bool free = id < szx && !hash_contains(H, hsize, id);
+                    const bool free = id < szx && !vis_contains(H, hsize, vbits, id);
                     const uint64_t m = ballot(free);
                     const uint32_t pos = nt + lanes_below(m);
                     if (free && pos < want) S[pos] = id;
@@ -974,16 +1021,16 @@ __global__ __launch_bounds__(64) void k_traverse(TravArgs p) {
             W[64u + lane] = w1;
             wave_sync();
             sort128(W);
-            hash_clear(H, hsize);
+            vis_clear(H, hsize, vbits);
             b = lane < R ? W[lane] : kCandSent;
             const uint64_t y = W[R + lane];
             for (uint32_t h = 0; h < 2; ++h) {
                 const uint64_t c = W[h * 64u + lane];
-                if (cvalid(c)) hash_insert(H, p.hsize, crow(c) - offx);
+                if (cvalid(c)) vis_insert(H, hsize, vbits, crow(c) - offx);
             }
             wave_sync();
             merge_into(A, L, y, 64u, nullptr);
-            hash_add_list(p, co, H, A, L, offx, offxn, n_lrow);
+            vis_add_list(p, O, H, A, L, kCandSent, offx, offxn, n_lrow);
         }
     }
 

@@ -76,10 +76,14 @@ extern "C" gf_status gf_search_noalloc(gf_index* ix, const float* queries, uint3
         GF_REQUIRE(!ix->C || (o->topc >= 1 && o->topc <= 4), GF_E_ARG, "topc must be in [1, 4]");
         GF_REQUIRE(so.entry_points || ix->entry_ref.n == R, GF_E_ARG,
                    "the index has no room for the reference's entry-point draw: pass entry_points");
-        const uint32_t hsize = gf::visited_slots(L + gf::kXSlots + 4 * R);
+        const uint32_t live = L + gf::kXSlots + 4 * R;
+        const gf::VisitedSet vs = gf::visited_set(ix->max_cell, live);
+        const uint32_t hsize = vs.words;
         const uint32_t Lpad = gf::round_up(L, 2);
         const uint32_t lds = gf::trav_lds_bytes(Lpad, hsize, ix->P);
-        GF_REQUIRE(lds <= 64 * 1024, GF_E_UNSUPPORTED, "L too large for the LDS budget");
+        // the limit on L is the hash table's, whichever form of the set runs
+        GF_REQUIRE(std::max(lds, gf::trav_lds_bytes(Lpad, gf::visited_slots(live), ix->P)) <= 64 * 1024, GF_E_UNSUPPORTED,
+                   "L too large for the LDS budget");
 
         // Sections, in the order gf_batch_create and the stage calls make them.
         const uint32_t Qp = gf::round_up(Q, 16);
@@ -205,6 +209,7 @@ extern "C" gf_status gf_search_noalloc(gf_index* ix, const float* queries, uint3
         t.counters = s.counters;
         t.a = a; t.P = P; t.R = R; t.E = ix->E; t.L = L; t.K = K; t.rl = rl;
         t.hsize = hsize;
+        t.vbits = vs.bits;
         t.offl = gf::trav_offsets_in_lds(ix->P) ? 1u : 0u;
         t.Lpad = Lpad;
         gf::SchedArgs sa{};

@@ -239,6 +239,7 @@ struct gf_index {
     bool ref_ties = false;   // stage B: equal cell scores in the reference's network order
     gf::RowShape rs{};
     uint32_t rowbytes = 0, Cp = 0, Dp = 0;
+    uint32_t max_cell = 0;   // points of the largest cell
     std::vector<uint32_t> offset_h, grid_h;
     DevBuf<char> vec;
     DevBuf<float> attrs, l_q, r_q, cnorm;

@@ -817,10 +817,14 @@ void stream_search(gf_batch& b, const gf_search_opts& o, uint32_t* ids, float* d
     if (b.out_ids.n < size_t(Q) * K) { b.out_ids.alloc(size_t(Q) * K); b.out_dist.alloc(size_t(Q) * K); }
     if (b.counters.n < size_t(Q) * GF_NCOUNTERS) b.counters.alloc(size_t(Q) * GF_NCOUNTERS);
 
-    const uint32_t hsize = visited_slots(L + kXSlots + 4 * R);
+    const uint32_t live = L + kXSlots + 4 * R;
+    const VisitedSet vs = visited_set(ix.max_cell, live);
+    const uint32_t hsize = vs.words;
     const uint32_t Lpad = round_up(L, 2);
     const uint32_t lds = trav_lds_bytes(Lpad, hsize, Bm);
-    GF_REQUIRE(lds <= 64 * 1024, GF_E_UNSUPPORTED, "L too large for the LDS budget");
+    // the limit on L is the hash table's, whichever form of the set runs
+    GF_REQUIRE(std::max(lds, trav_lds_bytes(Lpad, visited_slots(live), Bm)) <= 64 * 1024, GF_E_UNSUPPORTED,
+               "L too large for the LDS budget");
 
     TravArgs base{};
     base.rowbytes = ix.rowbytes;
@@ -839,6 +843,7 @@ void stream_search(gf_batch& b, const gf_search_opts& o, uint32_t* ids, float* d
     base.counters = b.s_ctr.p;
     base.a = ix.a; base.R = R; base.E = ix.E; base.L = L; base.K = K; base.rl = o.rl;
     base.hsize = hsize;
+    base.vbits = vs.bits;
     base.offl = trav_offsets_in_lds(Bm) ? 1u : 0u;   // lds holds Bm + 1 >= B + 1 offsets
     base.Lpad = Lpad;
     uint32_t* tot = b.tot.p;
