@@ -1182,6 +1182,14 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         if (gemm_h && b->hover.n < Q) b->hover.alloc(Q);
         if (!b->bf_all && b->bfmask.n < size_t(Q) * ix->P) b->bfmask.alloc(size_t(Q) * ix->P);
     }
+    gf::BfSplit split;
+    if (!sched_bf) {
+        split.cap = gf::bf_split_cap(Q, uint32_t(ix->ncu));
+        if (b->bfs_keys.n < size_t(split.cap) * K) b->bfs_keys.alloc(size_t(split.cap) * K);
+        if (b->bfs_cnt.n < split.cap) b->bfs_cnt.alloc(split.cap);
+        split.keys = b->bfs_keys.p;
+        split.cnt = b->bfs_cnt.p;
+    }
     // events: [0] search start, [1] after traversal, [2] end, [3..4] around the MFMA kernel alone
     // Device timestamps (wall clock, kernels on the stream, so that they
     // time a replayed graph too): [0] search start, [1] after traversal,
@@ -1414,7 +1422,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         } else {
             gf::TravArgs ab = a;
             ab.srange = tot + 14;
-            GF_HIP(gf::launch_bruteforce(ix->rs, ab, Q, st));
+            GF_HIP(gf::launch_bruteforce(ix->rs, ab, Q, st, split));
         }
         enqueue_copies(false);
     };
@@ -1435,7 +1443,8 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
                             uint64_t(uintptr_t(b->cells.p)), uint64_t(uintptr_t(b->gbound.p)),
                             uint64_t(uintptr_t(b->scnt.p)), uint64_t(uintptr_t(b->rq.p)),
                             uint64_t(uintptr_t(b->bcnt.p)), uint64_t(uintptr_t(b->h_tot.p)),
-                            uint64_t(uintptr_t(b->stamps.p)), uint64_t(uintptr_t(b->h_stamps.p))};
+                            uint64_t(uintptr_t(b->stamps.p)), uint64_t(uintptr_t(b->h_stamps.p)),
+                            uint64_t(uintptr_t(split.keys)), uint64_t(uintptr_t(split.cnt))};
     std::vector<uint64_t> gkey(std::begin(key), std::end(key));
     uint32_t ppf = 0;
     std::memcpy(&ppf, &pend_pf, sizeof(ppf));

@@ -447,7 +447,23 @@ hipError_t launch_fullgraph(const RowShape& rs, const TravArgs& a, uint32_t lds_
 hipError_t launch_assemble_full(const uint32_t* graph, const uint32_t* cross, const uint32_t* offset,
                                 const uint32_t* rowcell, uint32_t N, uint32_t P, uint32_t R, uint32_t E, uint32_t FE,
                                 uint32_t* out, hipStream_t st);
-hipError_t launch_bruteforce(const RowShape& rs, const TravArgs& a, uint32_t grid, hipStream_t st);
+// Gather brute force of fewer queries than the chip holds waves: each
+// query's rows in min(cap / queries, kBfSplitMax) parts, a wave each.  cap
+// (0: one wave per query) is the workgroups of the launch and the parts that
+// the arrays hold: keys cap * K, cnt cap.
+constexpr uint32_t kBfSplitMax = 128;
+constexpr uint32_t kBfSplitWaves = 16;   // waves per CU that a launch is cut into
+struct BfSplit {
+    uint64_t* keys = nullptr;
+    uint32_t* cnt = nullptr;
+    uint32_t cap = 0;
+};
+inline uint32_t bf_split_cap(uint32_t Q, uint32_t ncu) {
+    const uint64_t most = uint64_t(Q) * kBfSplitMax, fill = uint64_t(ncu) * kBfSplitWaves;
+    return uint32_t(most < fill ? most : fill);
+}
+hipError_t launch_bruteforce(const RowShape& rs, const TravArgs& a, uint32_t grid, hipStream_t st,
+                             const BfSplit& sp = {});
 hipError_t launch_fill_results(uint32_t* ids, float* dist, uint32_t n, hipStream_t st);
 hipError_t launch_bf_i8(const BfGemmArgs& a, uint32_t ncu, hipStream_t st);   // grid: ncu x resident workgroups per CU
 hipError_t launch_bf_final(const BfFinalArgs& a, uint32_t grid, hipStream_t st);

@@ -1545,53 +1545,56 @@ __global__ void k_assemble_full(const uint32_t* graph, const uint32_t* cross, co
 // Filtered brute force over the query's cells (gpu_graph.cu:3788-4022): an
 // attribute scan of each cell's contiguous rows, compaction of the passing
 // rows, distance evaluation and a wave-held top-K keyed by (distance, row).
+// Merges survivors c (one per lane, sentinels elsewhere) into the top-K.
+__device__ __forceinline__ void bf_merge_top(uint64_t c, uint32_t K, uint64_t& top, uint64_t* T) {
+    const uint32_t lane = lane_id();
+    const bool surv = ckey(c) < ckey(readlane64(top, K - 1));
+    const uint64_t sm = ballot(surv);
+    if (sm == 0) return;
+    const uint64_t kc = ckey(c), kt = ckey(top);
+    uint32_t rs = 0, rt = lane;
+    // ranks in the merged order, ties to the top entry, then to the lower
+    // lane: a permutation even if a key repeats
+    for (uint64_t m = sm; m; m &= m - 1) {
+        const uint32_t j = __builtin_ctzll(m);
+        const uint64_t kk = readlane64(kc, j);
+        rs += kk < kc || (kk == kc && j < lane);
+        rt += kk < kt;
+    }
+    for (uint32_t t = 0; t < K; ++t) rs += readlane64(kt, t) <= kc;
+    wave_sync();
+    if (surv && rs < K) T[rs] = c;
+    if (lane < K && rt < K) T[rt] = top;
+    wave_sync();
+    top = lane < K ? T[lane] : kCandSent;
+}
+
 // Exact distances of the rows S[0..nrows) to the query, merged into the
 // top-K (lane t < K: t-th best by (distance, row)).
 template <int VT, int LPR, int CPL>
 __device__ void bf_flush(const QReg<VT, LPR, CPL>& qv, const TravArgs& p, uint32_t* S, uint32_t nrows,
                          uint64_t& top, uint64_t* T) {
-    const uint32_t lane = lane_id(), K = p.K;
-    {
-        for (uint32_t base = 0; base < nrows; base += 64u) {
-            const uint32_t nb = nrows - base < 64u ? nrows - base : 64u;
-            const bool mine = lane < nb;
-            const uint32_t row = mine ? S[base + lane] : 0u;
-            float d = 0.0f;
-            eval_rows<VT, LPR, CPL>(qv, p.vec, p.rowbytes, p.nch, S + base, nb,
-                                     mine ? lane : 0xFFFFFFFFu, d);
-            const uint64_t c = mine ? make_cand(d, row, true) : kCandSent;
-            const uint64_t thr = ckey(readlane64(top, K - 1));
-            const bool surv = mine && ckey(c) < thr;
-            const uint64_t sm = ballot(surv);
-            if (sm == 0) continue;
-            const uint64_t kc = ckey(c), kt = ckey(top);
-            uint32_t rs = 0, rt = lane;
-            // ranks in the merged order, ties to the top entry, then to the
-            // lower lane: a permutation even if a key repeats
-            for (uint64_t m = sm; m; m &= m - 1) {
-                const uint32_t j = __builtin_ctzll(m);
-                const uint64_t kk = readlane64(kc, j);
-                rs += kk < kc || (kk == kc && j < lane);
-                rt += kk < kt;
-            }
-            for (uint32_t t = 0; t < K; ++t) rs += readlane64(kt, t) <= kc;
-            wave_sync();
-            if (surv && rs < K) T[rs] = c;
-            if (lane < K && rt < K) T[rt] = top;
-            wave_sync();
-            top = lane < K ? T[lane] : kCandSent;
-        }
+    const uint32_t lane = lane_id();
+    for (uint32_t base = 0; base < nrows; base += 64u) {
+        const uint32_t nb = nrows - base < 64u ? nrows - base : 64u;
+        const bool mine = lane < nb;
+        const uint32_t row = mine ? S[base + lane] : 0u;
+        float d = 0.0f;
+        eval_rows<VT, LPR, CPL>(qv, p.vec, p.rowbytes, p.nch, S + base, nb, mine ? lane : 0xFFFFFFFFu, d);
+        bf_merge_top(mine ? make_cand(d, row, true) : kCandSent, p.K, top, T);
     }
 }
 
-// Filtered brute force of query q over the first little[q] cells of its
-// list: the passing rows are gathered 64 at a time and ranked exactly.
-// Results and counters are written for q.
+// Filtered brute force of query q over part `part` of `np` equal parts of
+// the rows of the first little[q] cells of its list: the passing rows are
+// gathered 64 at a time and ranked exactly (lane t < K of top: t-th best).
+// Returns the rows that passed; nscan: the rows of all parts.
 template <int VT, int LPR, int CPL>
-__device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64_t* T) {
+__device__ uint32_t bf_scan_rows(const TravArgs& p, uint32_t q, uint32_t part, uint32_t np, uint32_t* S, uint64_t* T,
+                                 uint64_t& top, uint32_t& nscan) {
     constexpr uint32_t U = 4;                 // 64-row chunks scanned per step (S holds 64 U + 64)
     const uint32_t lane = lane_id();
-    const uint32_t K = p.K, P = p.P;
+    const uint32_t P = p.P;
     QReg<VT, LPR, CPL> qv;
     load_query<VT, LPR, CPL>(qv, p.queries + size_t(q) * p.qbytes, p.nch);
     float lo[kMaxAttr], hi[kMaxAttr];
@@ -1600,18 +1603,26 @@ __device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64
         lo[d] = d < p.a ? p.lo[size_t(q) * p.a + d] : 0.0f;
         hi[d] = d < p.a ? p.hi[size_t(q) * p.a + d] : 0.0f;
     }
-    uint64_t top = kCandSent;                 // lane t < K: t-th best
-    uint32_t n_scan = 0, n_pass = 0;
+    top = kCandSent;
+    uint32_t n_pass = 0;
     const uint32_t* cl = p.cells + size_t(q) * P;
     const uint32_t lit = p.little[q];
-    uint32_t ns = 0;
-    auto flush = [&](uint32_t nrows) { bf_flush<VT, LPR, CPL>(qv, p, S, nrows, top, T); };
-
-    for (uint32_t g = 0; g < lit; ++g) {
+    uint32_t total = 0;
+    for (uint32_t i = lane; i < lit; i += 64u) total += p.offset[cl[i] + 1] - p.offset[cl[i]];
+#pragma unroll
+    for (uint32_t o = 32; o; o >>= 1) total += uint32_t(__shfl_xor(int(total), int(o)));
+    nscan = total;
+    // this part's rows, as positions in the concatenation of the cells
+    const uint32_t r0 = uint32_t(uint64_t(total) * part / np), r1 = uint32_t(uint64_t(total) * (part + 1u) / np);
+    uint32_t ns = 0, before = 0;
+    for (uint32_t g = 0; g < lit && before < r1; ++g) {
         const uint32_t cc = cl[g];
-        const uint32_t off = p.offset[cc], end = p.offset[cc + 1];
-        n_scan += end - off;
-        for (uint32_t base = off; base < end; base += 64u * U) {
+        const uint32_t off = p.offset[cc], size = p.offset[cc + 1] - off;
+        const uint32_t b0 = r0 > before ? r0 - before : 0u, b1 = r1 - before < size ? r1 - before : size;
+        before += size;
+        if (b0 >= b1) continue;
+        const uint32_t end = off + b1;
+        for (uint32_t base = off + b0; base < end; base += 64u * U) {
             bool ps[U];
 #pragma unroll
             for (uint32_t u = 0; u < U; ++u) {
@@ -1627,7 +1638,7 @@ __device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64
             wave_sync();
             if (ns >= 64u) {
                 const uint32_t full = ns & ~63u;
-                flush(full);
+                bf_flush<VT, LPR, CPL>(qv, p, S, full, top, T);
                 const uint32_t rest = ns - full;
                 const uint32_t tail = lane < rest ? S[full + lane] : 0u;
                 wave_sync();
@@ -1638,7 +1649,15 @@ __device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64
             }
         }
     }
-    if (ns) { flush(ns); n_pass += ns; }
+    if (ns) {
+        bf_flush<VT, LPR, CPL>(qv, p, S, ns, top, T);
+        n_pass += ns;
+    }
+    return n_pass;
+}
+
+__device__ __forceinline__ void bf_write_query(const TravArgs& p, uint32_t q, uint64_t top, uint32_t n_scan, uint32_t n_pass) {
+    const uint32_t lane = lane_id(), K = p.K;
     if (lane < K) {
         p.out_ids[size_t(q) * K + lane] = cvalid(top) ? p.gidx[crow(top)] : GF_NO_RESULT;
         p.out_dist[size_t(q) * K + lane] = cdist(top);
@@ -1652,17 +1671,92 @@ __device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64
         ctr[C_LROW] = 0;
         ctr[C_SCAN] = n_scan;
         ctr[C_PASS] = n_pass;
-        ctr[C_ROUTE] = lit ? 2u : 0u;
+        ctr[C_ROUTE] = p.little[q] ? 2u : 0u;
     }
 }
 
+// Filtered brute force of query q by one wave: results and counters.
 template <int VT, int LPR, int CPL>
-__global__ __launch_bounds__(64) void k_bruteforce(TravArgs p) {
+__device__ void bf_scan_query(const TravArgs& p, uint32_t q, uint32_t* S, uint64_t* T) {
+    uint64_t top;
+    uint32_t n_scan;
+    const uint32_t n_pass = bf_scan_rows<VT, LPR, CPL>(p, q, 0, 1, S, T, top, n_scan);
+    bf_write_query(p, q, top, n_scan, n_pass);
+}
+
+// Parts that each of nq queries is cut into.
+__device__ __forceinline__ uint32_t bf_split_parts(const BfSplit& sp, uint32_t nq) {
+    const uint32_t np = sp.cap / nq;
+    return np < 1u ? 1u : np < kBfSplitMax ? np : kBfSplitMax;
+}
+
+// One wave per part of a query.  A query alone on one wave took 290 us over
+// 100k x 128 fp32 rows (5 % passing) on an otherwise idle chip, and 43
+// queries together 1.54 ms (their longest); cut into parts they take 24
+// and 70 us, merge included.  np follows the number of queries on this route,
+// which only the device knows.  Each part leaves its top K and its count in
+// the split's arrays for k_bf_merge; merging in the part that finishes last
+// needed a device-scope fence per part, whose L2 write-backs took longer
+// (320 us for the 43 queries) than the launch it saved.
+template <int VT, int LPR, int CPL>
+__global__ __launch_bounds__(64) void k_bruteforce(TravArgs p, BfSplit sp) {
     __shared__ uint32_t S[64 * 4 + 64];
     __shared__ uint64_t T[64];
-    const uint32_t si = p.srange[0] + blockIdx.x;
-    if (si >= p.srange[1]) return;
-    bf_scan_query<VT, LPR, CPL>(p, p.sched[si], S, T);
+    const uint32_t begin = p.srange[0], nq = p.srange[1] - begin;
+    if (nq == 0) return;
+    const uint32_t np = bf_split_parts(sp, nq);
+    const uint32_t si = blockIdx.x / np, part = blockIdx.x % np;
+    if (si >= nq) return;
+    const uint32_t q = p.sched[begin + si];
+    if (np == 1) {
+        bf_scan_query<VT, LPR, CPL>(p, q, S, T);
+        return;
+    }
+    uint64_t top;
+    uint32_t n_scan;
+    const uint32_t n_pass = bf_scan_rows<VT, LPR, CPL>(p, q, part, np, S, T, top, n_scan);
+    const uint32_t lane = lane_id(), K = p.K;
+    const size_t at = size_t(si) * np + part;
+    if (lane < K) sp.keys[at * K + lane] = top;
+    if (lane == 0) sp.cnt[at] = n_pass;
+}
+
+// One wave per query that k_bruteforce cut into parts: the K best of the
+// parts' keys, results and counters.
+__global__ __launch_bounds__(64) void k_bf_merge(TravArgs p, BfSplit sp) {
+    __shared__ uint64_t T[64];
+    const uint32_t begin = p.srange[0], nq = p.srange[1] - begin;
+    if (blockIdx.x >= nq) return;
+    const uint32_t np = bf_split_parts(sp, nq);
+    if (np == 1) return;
+    const uint32_t si = blockIdx.x, q = p.sched[begin + si], lane = lane_id(), K = p.K, n = np * K;
+    uint32_t pass = 0, scan = 0;
+    for (uint32_t i = lane; i < np; i += 64u) pass += sp.cnt[size_t(si) * np + i];
+    for (uint32_t i = lane; i < p.little[q]; i += 64u) {
+        const uint32_t c = p.cells[size_t(q) * p.P + i];
+        scan += p.offset[c + 1] - p.offset[c];
+    }
+#pragma unroll
+    for (uint32_t o = 32; o; o >>= 1) {
+        pass += uint32_t(__shfl_xor(int(pass), int(o)));
+        scan += uint32_t(__shfl_xor(int(scan), int(o)));
+    }
+    const uint64_t* keys = sp.keys + size_t(si) * n;
+    uint64_t top = kCandSent;
+    constexpr uint32_t U = 8;
+    for (uint32_t base = 0; base < n; base += 64u * U) {
+        uint64_t c[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            // keys by rank, then part: the parts' best come first and most
+            // later chunks hold no key below the K-th
+            const uint32_t i = base + u * 64u + lane;
+            c[u] = i < n ? keys[size_t(i % np) * K + i / np] : kCandSent;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) bf_merge_top(c[u], K, top, T);
+    }
+    bf_write_query(p, q, top, scan, pass);
 }
 
 __global__ void k_fill_results(uint32_t* ids, float* dist, uint32_t n) {
@@ -4522,9 +4616,11 @@ hipError_t launch_full_t(const TravArgs& a, uint32_t lds, uint32_t grid, hipStre
     return hipGetLastError();
 }
 template <int VT, int LPR, int CPL>
-hipError_t launch_bf_t(const TravArgs& a, uint32_t grid, hipStream_t st) {
+hipError_t launch_bf_t(const TravArgs& a, uint32_t grid, const BfSplit& sp, hipStream_t st) {
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_bruteforce<VT, LPR, CPL>), dim3(grid), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((k_bruteforce<VT, LPR, CPL>), dim3(sp.cap > grid ? sp.cap : grid), dim3(64), 0, st, a, sp);
+    // two queries' worth of parts or more: some query may have been cut
+    if (sp.cap > 1) hipLaunchKernelGGL(k_bf_merge, dim3(grid < sp.cap ? grid : sp.cap), dim3(64), 0, st, a, sp);
     return hipGetLastError();
 }
 
@@ -4686,8 +4782,9 @@ hipError_t launch_assemble_full(const uint32_t* graph, const uint32_t* cross, co
     return hipGetLastError();
 }
 
-hipError_t launch_bruteforce(const RowShape& rs, const TravArgs& a, uint32_t grid, hipStream_t st) {
-#define CALL_B(V, L_, C_) launch_bf_t<V, L_, C_>(a, grid, st)
+hipError_t launch_bruteforce(const RowShape& rs, const TravArgs& a, uint32_t grid, hipStream_t st,
+                             const BfSplit& sp) {
+#define CALL_B(V, L_, C_) launch_bf_t<V, L_, C_>(a, grid, sp, st)
     GF_DISPATCH(CALL_B);
 #undef CALL_B
     return hipErrorInvalidValue;

@@ -88,12 +88,16 @@ extern "C" gf_status gf_search_noalloc(gf_index* ix, const float* queries, uint3
         // Sections, in the order gf_batch_create and the stage calls make them.
         const uint32_t Qp = gf::round_up(Q, 16);
         Carve cv{nullptr};
+        // the brute force in parts, where its arrays fit beside the batch
+        uint32_t split_cap = gf::bf_split_cap(Q, uint32_t(ix->ncu));
         auto layout = [&](Carve& c) {
             struct {
                 float *qf32, *lo, *hi, *qnorm, *out_dist;
                 uint16_t *q16v, *q16;
                 uint32_t *cells, *counts, *little, *selcount, *cellq, *ccount, *cstart, *cfill, *topk, *sched,
                     *tot, *entry, *out_ids, *counters;
+                uint64_t* bfs_keys;
+                uint32_t* bfs_cnt;
             } s{};
             s.qf32 = c.take<float>(size_t(Q) * D);
             s.lo = c.take<float>(size_t(Q) * a);
@@ -120,11 +124,18 @@ extern "C" gf_status gf_search_noalloc(gf_index* ix, const float* queries, uint3
             s.out_ids = c.take<uint32_t>(size_t(Q) * K);
             s.out_dist = c.take<float>(size_t(Q) * K);
             s.counters = c.take<uint32_t>(size_t(Q) * GF_NCOUNTERS);
+            s.bfs_keys = c.take<uint64_t>(size_t(split_cap) * K);
+            s.bfs_cnt = c.take<uint32_t>(split_cap);
             return s;
         };
         {
             Carve probe{nullptr};
             (void)layout(probe);
+            if (probe.used > kScratchBytes) {
+                split_cap = 0;
+                probe = Carve{nullptr};
+                (void)layout(probe);
+            }
             GF_REQUIRE(probe.used <= kScratchBytes, GF_E_UNSUPPORTED,
                        "batch needs " + std::to_string(probe.used) + " bytes of scratch, more than the " +
                            std::to_string(kScratchBytes) + " of gf_search_noalloc: use fewer queries");
@@ -236,7 +247,11 @@ extern "C" gf_status gf_search_noalloc(gf_index* ix, const float* queries, uint3
         }
         gf::TravArgs tb = t;
         tb.srange = s.tot + 14;
-        GF_HIP(gf::launch_bruteforce(ix->rs, tb, Q, st));
+        gf::BfSplit split;
+        split.keys = s.bfs_keys;
+        split.cnt = s.bfs_cnt;
+        split.cap = split_cap;
+        GF_HIP(gf::launch_bruteforce(ix->rs, tb, Q, st, split));
         GF_HIP(hipMemcpyAsync(ids, s.out_ids, size_t(Q) * K * 4, hipMemcpyDeviceToHost, st));
         if (dists) GF_HIP(hipMemcpyAsync(dists, s.out_dist, size_t(Q) * K * 4, hipMemcpyDeviceToHost, st));
         GF_HIP(hipStreamSynchronize(st));

@@ -420,6 +420,8 @@ struct gf_batch {
     DevBuf<uint16_t> q16, q16v;
     DevBuf<float> qi8q;   // GF_VEC_I8Q: query rows [c | s], c_d = fma(s_d, z_d, q_d)
     DevBuf<float> qnf, heps;   // float MFMA brute force: |q|^2 of the query as the rows hold it, bound of |d' - d|
+    DevBuf<uint64_t> bfs_keys;  // gather brute force in parts (gf::BfSplit)
+    DevBuf<uint32_t> bfs_cnt;
     DevBuf<uint32_t> hover;     // fp16 brute force: queries whose kept keys may miss a candidate
     DevBuf<uint32_t> cells, counts, little, selcount, cellq, ccount, cstart, cfill, topk;
     DevBuf<uint32_t> out_ids, counters, sched, entry, gbound;
