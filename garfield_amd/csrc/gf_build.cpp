@@ -395,57 +395,59 @@ void optimize_graphs(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t
     std::vector<uint32_t> offset(P + 1, 0);
     for (uint32_t c = 0; c < P; ++c) offset[c + 1] = offset[c] + cell_size[c];
     GF_REQUIRE(offset[P] == N, GF_E_ARG, "cell sizes do not add up to N");
-    for (uint32_t c = 0; c < P; ++c)
-        for (size_t k = size_t(offset[c]) * I; k < size_t(offset[c + 1]) * I; ++k)
-            GF_REQUIRE(knn[k] < cell_size[c], GF_E_FORMAT, "kNN graph holds an id beyond its cell");
-    std::vector<uint32_t> ord(size_t(N) * I);
-    {
-        GF_HIP(hipSetDevice(device));
-        hipStream_t st = nullptr;
-        GF_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        struct StreamGuard {
-            hipStream_t s;
-            ~StreamGuard() { (void)hipStreamDestroy(s); }
-        } guard{st};
-        DevBuf<uint32_t> dk, doff, dout;
-        dk.upload(knn, size_t(N) * I);
-        doff.upload(offset);
-        dout.alloc(size_t(N) * I);
-        GF_HIP(launch_prune(dk.p, N, I, doff.p, P, dout.p, st));
-        GF_HIP(hipMemcpyAsync(ord.data(), dout.p, ord.size() * 4, hipMemcpyDeviceToHost, st));
-        GF_HIP(hipStreamSynchronize(st));
-    }
-    // Reverse edges: for every rank k of the pruned lists (their first R
-    // entries), in node order, the edge A -> B adds A to B's reverse list
-    // (at most R, a node never lists itself).  Each row then keeps the first
-    // R / 2 pruned edges, appends reverse edges, then the rest of its
-    // reordered list, each id once; a row still short (a cell of fewer than
-    // R + 1 points) repeats its first entry.
-    const uint32_t keep = R / 2;
-    std::vector<uint32_t> mark;
     for (uint32_t c = 0; c < P; ++c) {
-        const uint32_t off = offset[c], n = cell_size[c];
-        std::vector<uint32_t> rev(size_t(n) * R), rcnt(n, 0);
-        for (uint32_t k = 0; k < R; ++k)
-            for (uint32_t a = 0; a < n; ++a) {
-                const uint32_t b = ord[(size_t(off) + a) * I + k];
-                if (b != a && rcnt[b] < R) rev[size_t(b) * R + rcnt[b]++] = a;
-            }
-        mark.assign(n, 0);
-        for (uint32_t a = 0; a < n; ++a) {
-            const uint32_t* o = &ord[(size_t(off) + a) * I];
-            uint32_t* g = graphs + (size_t(off) + a) * R;
-            const uint32_t stamp = a + 1;
-            uint32_t m = 0;
-            auto put = [&](uint32_t x) {
-                if (m < R && mark[x] != stamp) { mark[x] = stamp; g[m++] = x; }
-            };
-            for (uint32_t k = 0; k < keep; ++k) put(o[k]);
-            for (uint32_t t = 0; t < rcnt[a]; ++t) put(rev[size_t(a) * R + t]);
-            for (uint32_t k = keep; k < I; ++k) put(o[k]);
-            for (; m < R; ++m) g[m] = g[0];
-        }
+        uint32_t most = 0;   // a maximum, not a test per id: it vectorises
+        for (size_t k = size_t(offset[c]) * I; k < size_t(offset[c + 1]) * I; ++k) most = std::max(most, knn[k]);
+        GF_REQUIRE(!cell_size[c] || most < cell_size[c], GF_E_FORMAT, "kNN graph holds an id beyond its cell");
     }
+    GF_HIP(hipSetDevice(device));
+    hipStream_t st = nullptr;
+    GF_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    struct StreamGuard {
+        hipStream_t s;
+        ~StreamGuard() { (void)hipStreamDestroy(s); }
+    } guard{st};
+    DevBuf<uint32_t> dk, doff, dord, dout, dcnt;
+    DevBuf<uint64_t> dstart, dpairs;
+    DevBuf<unsigned long long> dused;
+    dk.upload(knn, size_t(N) * I);
+    doff.upload(offset);
+    dord.alloc(size_t(N) * I);
+    dout.alloc(size_t(N) * R);
+    GF_HIP(launch_prune(dk.p, N, I, doff.p, P, dord.p, st));
+    // Reverse edges and the final rows, whole cells at a time: as many cells
+    // as keep the pairs' scratch within kRevPairs entries (one cell at least).
+    constexpr size_t kRevPairs = size_t(1) << 28;
+    std::vector<uint32_t> cut{0};   // first cell of each group
+    uint32_t most = 0;
+    for (uint32_t c = 1; c <= P; ++c) {
+        const size_t rows = offset[c] - offset[cut.back()];
+        if (rows * R > kRevPairs && c - 1 > cut.back()) cut.push_back(c - 1);
+    }
+    cut.push_back(P);
+    for (size_t g = 0; g + 1 < cut.size(); ++g) most = std::max(most, offset[cut[g + 1]] - offset[cut[g]]);
+    dcnt.alloc(most);
+    dstart.alloc(most);
+    dpairs.alloc(size_t(most) * R);
+    dused.alloc(1);
+    RevArgs ra{};
+    ra.ord = dord.p;
+    ra.offset = doff.p;
+    ra.I = I;
+    ra.R = R;
+    ra.P = P;
+    ra.cnt = dcnt.p;
+    ra.start = dstart.p;
+    ra.used = dused.p;
+    ra.pairs = dpairs.p;
+    ra.out = dout.p;
+    for (size_t g = 0; g + 1 < cut.size(); ++g) {
+        ra.row0 = offset[cut[g]];
+        ra.n = offset[cut[g + 1]] - ra.row0;
+        GF_HIP(launch_rev_edges(ra, st));
+    }
+    GF_HIP(hipMemcpyAsync(graphs, dout.p, size_t(N) * R * 4, hipMemcpyDeviceToHost, st));
+    GF_HIP(hipStreamSynchronize(st));
     if (ms) *ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 

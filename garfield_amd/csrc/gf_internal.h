@@ -291,6 +291,21 @@ hipError_t launch_rerank(const RerankArgs& a, uint32_t D, uint32_t nlists, hipSt
 // rank) order.  I <= 64.
 hipError_t launch_prune(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t* offset, uint32_t P,
                         uint32_t* out, hipStream_t st);
+// Graph optimisation, second step, on rows [row0, row0 + n) of whole cells:
+// reverse edges of the first R entries of the reordered lists ord (rows of I)
+// and the final rows of R ids.  Scratch: cnt and start (n each), pairs (n *
+// R), used (one counter).
+struct RevArgs {
+    const uint32_t* ord;
+    const uint32_t* offset;    // P + 1 first rows of the cells
+    uint32_t I, R, P, row0, n;
+    uint32_t* cnt;
+    uint64_t* start;
+    unsigned long long* used;
+    uint64_t* pairs;
+    uint32_t* out;             // N * R
+};
+hipError_t launch_rev_edges(const RevArgs& a, hipStream_t st);
 // k-means update: cnt and fill (C each) must start at zero; start (C) and
 // mem (N) are scratch; centres (C x Dp u8) are rewritten where a cluster
 // has members.

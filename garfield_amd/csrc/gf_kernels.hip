@@ -4470,17 +4470,39 @@ __global__ __launch_bounds__(256) void k_kmeans_mean(const uint8_t* vec, uint32_
     }
 }
 
+// Small id -> value table in LDS (linear probing over 2^k slots, at most
+// half to two thirds full): the slot of `id`, claimed if it is new.
+template <uint32_t SLOTS>
+__device__ __forceinline__ uint32_t id_slot(uint32_t* keys, uint32_t id) {
+    uint32_t h = (id * 2654435761u) >> (32 - __builtin_ctz(SLOTS));
+    for (uint32_t i = 0; i < SLOTS; ++i) {
+        const uint32_t old = atomicCAS(&keys[h], kEmpty, id);
+        if (old == kEmpty || old == id) return h;
+        h = (h + 1u) & (SLOTS - 1u);
+    }
+    return 0;
+}
+
 // Rank-based reordering of a kNN graph, the first step of CAGRA's graph
 // optimisation (Ootomo et al., "CAGRA: Highly Parallel Graph Construction and
 // Approximate Nearest Neighbor Search for GPUs", ICDE 2024): the edge A -> D
 // at rank k of A's list has a detour through every B at a rank below k in A's
 // list that lists D at a rank below k; A's edges are written in ascending
-// (detours, rank) order.  One wave per row: A's I neighbour lists are staged
-// in LDS (I x I ids) and lane k counts the detours of edge k.  Rows are
-// cell-major and ids cell-local (row = offset[cell] + id).
+// (detours, rank) order.  One wave per row.  A's ids go into an LDS table
+// with their ranks, and each neighbour's list passes by once, a lane per
+// entry, eight lists in flight: an entry found in the table at a rank above
+// both its own and its list's sets its list's bit in that edge's mask
+// (a list that repeats an id sets it once).  Bound by instruction issue,
+// about 25 per list.  Staging the I lists in LDS and comparing every edge
+// with every entry took I^3 / 3 compares: 22.1 ms for 200k rows of 64,
+// 1.1 ms this way.  A row that repeats an id (a cell smaller than the list)
+// counts each of the equal edges: it takes the compares.
 __global__ __launch_bounds__(64) void k_prune(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t* offset,
                                               uint32_t P, uint32_t* out) {
-    extern __shared__ uint32_t nl[];   // I x I
+    constexpr uint32_t SLOTS = 256, B = 8;
+    __shared__ uint32_t keys[SLOTS];
+    __shared__ uint32_t rank[SLOTS];
+    __shared__ unsigned long long mask[64];
     const uint32_t lane = lane_id(), row = blockIdx.x;
     if (row >= N) return;
     uint32_t lo = 0, hi = P;           // the cell: last c with offset[c] <= row
@@ -4490,35 +4512,198 @@ __global__ __launch_bounds__(64) void k_prune(const uint32_t* knn, uint32_t N, u
     }
     const uint32_t base = offset[lo];
     const uint32_t d = lane < I ? knn[size_t(row) * I + lane] : kEmpty;
-    for (uint32_t k = 0; k < I; ++k) {
-        const uint32_t b = readlane32(d, k);
-        if (lane < I) nl[k * I + lane] = knn[(size_t(base) + b) * I + lane];
+    for (uint32_t i = lane; i < SLOTS; i += 64u) {
+        keys[i] = kEmpty;
+        rank[i] = kEmpty;
     }
-    __syncthreads();
-    uint32_t cnt = 0;
+    mask[lane] = 0;
+    wave_sync();
+    bool own = true;
     if (lane < I) {
-        for (uint32_t kb = 0; kb < lane; ++kb) {
-            const uint32_t* lb = nl + kb * I;
-            bool f = false;
-            for (uint32_t j = 0; j < lane; ++j) f = f || lb[j] == d;
-            cnt += f ? 1u : 0u;
+        const uint32_t sl = id_slot<SLOTS>(keys, d);
+        own = atomicMin(&rank[sl], lane) == kEmpty;
+    }
+    wave_sync();
+    const bool dup = ballot(lane < I && !own) != 0;
+    for (uint32_t k0 = 0; k0 < I; k0 += B) {
+        uint32_t e[B];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) {
+            e[u] = kEmpty;
+            if (k0 + u < I) {
+                const uint32_t b = readlane32(d, k0 + u);
+                if (lane < I) e[u] = knn[(size_t(base) + b) * I + lane];
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) {
+            if (k0 + u >= I) break;
+            const uint32_t kb = k0 + u;
+            if (!dup) {
+                if (lane < I) {
+                    uint32_t h = (e[u] * 2654435761u) >> (32 - __builtin_ctz(SLOTS));
+                    uint32_t key = keys[h];
+                    while (key != e[u] && key != kEmpty) {   // empty slots end every probe: at most 64 of 256 are taken
+                        h = (h + 1u) & (SLOTS - 1u);
+                        key = keys[h];
+                    }
+                    if (key == e[u]) {
+                        const uint32_t k = rank[h];
+                        if (k > kb && k > lane) atomicOr(&mask[k], 1ull << kb);
+                    }
+                }
+            } else {
+                for (uint32_t k = kb + 1u; k < I; ++k) {
+                    const uint32_t dk = readlane32(d, k);
+                    if (ballot(lane < k && e[u] == dk) != 0 && lane == 0) atomicOr(&mask[k], 1ull << kb);
+                }
+            }
         }
     }
+    wave_sync();
+    const uint32_t cnt = uint32_t(__popcll(mask[lane]));
+    const uint32_t ord = lane < I ? cnt << 6 | lane : kEmpty;   // (detours, rank), distinct
     uint32_t pos = 0;
-    for (uint32_t k = 0; k < I; ++k) {
-        const uint32_t ck = readlane32(cnt, k);
-        pos += (ck < cnt || (ck == cnt && k < lane)) ? 1u : 0u;
-    }
+    for (uint32_t k = 0; k < I; ++k) pos += readlane32(ord, k) < ord;
     if (lane < I) out[size_t(row) * I + pos] = d;
 }
 
+// Second step: reverse edges.  For every rank k of the reordered lists'
+// first R entries, in node order, the edge A -> B adds A to B's reverse list
+// (at most R, a node never lists itself).  k_rev_count counts the edges into
+// each node, k_rev_start gives each node a region of `pairs` (the regions'
+// order does not matter), k_rev_fill writes (k, A) there, and k_rev_merge
+// takes a node's R smallest pairs and writes its row.  Rows [row0, row0 +
+// n) of whole cells; ids are cell-local, offset the cells' first rows.
+__device__ __forceinline__ uint32_t cell_base(const uint32_t* offset, uint32_t P, uint32_t row) {
+    uint32_t lo = 0, hi = P;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (offset[mid] <= row) lo = mid; else hi = mid;
+    }
+    return offset[lo];
+}
+__global__ __launch_bounds__(256) void k_rev_count(RevArgs p) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= p.n) return;
+    const uint32_t row = p.row0 + i, base = cell_base(p.offset, p.P, row);
+    for (uint32_t k = 0; k < p.R; ++k) {
+        const uint32_t b = base + p.ord[size_t(row) * p.I + k];
+        if (b != row) atomicAdd(&p.cnt[b - p.row0], 1u);
+    }
+}
+__global__ __launch_bounds__(1024) void k_rev_start(RevArgs p) {
+    __shared__ uint32_t wsum[16];
+    __shared__ unsigned long long at;
+    const uint32_t i = blockIdx.x * 1024u + threadIdx.x;
+    const uint32_t v = i < p.n ? p.cnt[i] : 0u;
+    uint32_t total;   // edges into 1024 nodes: below 2^32 for cells of less than 2^32 / R points
+    const uint32_t ex = block_exclusive_scan(v, wsum, total);
+    if (threadIdx.x == 0) at = atomicAdd(p.used, (unsigned long long)total);
+    __syncthreads();
+    if (i < p.n) {
+        p.start[i] = at + ex;
+        p.cnt[i] = 0;   // k_rev_fill counts again
+    }
+}
+__global__ __launch_bounds__(256) void k_rev_fill(RevArgs p) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= p.n) return;
+    const uint32_t row = p.row0 + i, base = cell_base(p.offset, p.P, row);
+    for (uint32_t k = 0; k < p.R; ++k) {
+        const uint32_t b = base + p.ord[size_t(row) * p.I + k];
+        if (b == row) continue;
+        const uint32_t j = atomicAdd(&p.cnt[b - p.row0], 1u);
+        p.pairs[p.start[b - p.row0] + j] = uint64_t(k) << 32 | (row - base);
+    }
+}
+// One wave per node: the first R / 2 reordered edges, the reverse edges in
+// (rank, node) order, then the rest of the reordered list, each id once; a
+// row still short repeats its first entry.
+__global__ __launch_bounds__(64) void k_rev_merge(RevArgs p) {
+    constexpr uint32_t SLOTS = 256, T = 3;   // at most 32 + 64 + 64 entries
+    __shared__ uint32_t keys[SLOTS], first[SLOTS];
+    __shared__ uint64_t top_[64];
+    __shared__ uint32_t seq[64 * T];
+    const uint32_t i = blockIdx.x, lane = lane_id(), row = p.row0 + i, R = p.R, I = p.I, keep = R / 2u;
+    const uint32_t m = p.cnt[i];
+    const uint64_t* pr = p.pairs + p.start[i];
+    const uint32_t o = lane < I ? p.ord[size_t(row) * I + lane] : 0u;
+    uint64_t top = ~uint64_t(0);              // lane t < R: the t-th smallest pair
+    for (uint32_t s0 = 0; s0 < m; s0 += 64u) {
+        const uint64_t c = s0 + lane < m ? pr[s0 + lane] : ~uint64_t(0);
+        const bool surv = c < readlane64(top, R - 1u);
+        const uint64_t sm = ballot(surv);
+        if (!sm) continue;
+        uint32_t rs = 0, rt = lane;            // pairs are distinct
+        for (uint64_t x = sm; x; x &= x - 1) {
+            const uint64_t kk = readlane64(c, __builtin_ctzll(x));
+            rs += kk < c;
+            rt += kk < top;
+        }
+        if (s0)
+            for (uint32_t t = 0; t < R; ++t) rs += readlane64(top, t) < c;
+        wave_sync();
+        if (lane < R) top_[lane] = ~uint64_t(0);
+        wave_sync();
+        if (surv && rs < R) top_[rs] = c;
+        if (s0 && lane < R && rt < R) top_[rt] = top;
+        wave_sync();
+        top = lane < R ? top_[lane] : ~uint64_t(0);
+    }
+    const uint32_t nrev = m < R ? m : R, n = I + nrev;
+    for (uint32_t t = lane; t < SLOTS; t += 64u) {
+        keys[t] = kEmpty;
+        first[t] = kEmpty;
+    }
+    if (lane < I) seq[lane < keep ? lane : lane + nrev] = o;
+    if (lane < nrev) seq[keep + lane] = uint32_t(top);
+    wave_sync();
+    uint32_t id[T], sl[T];
+#pragma unroll
+    for (uint32_t t = 0; t < T; ++t) {
+        const uint32_t j = t * 64u + lane;
+        if (j < n) {
+            id[t] = seq[j];
+            sl[t] = id_slot<SLOTS>(keys, id[t]);
+            atomicMin(&first[sl[t]], j);
+        }
+    }
+    wave_sync();
+    uint32_t w = 0;
+    uint32_t* g = p.out + size_t(row) * R;
+#pragma unroll
+    for (uint32_t t = 0; t < T; ++t) {
+        const uint32_t j = t * 64u + lane;
+        const bool one = j < n && first[sl[t]] == j;
+        const uint64_t mm = ballot(one);
+        const uint32_t pos = w + lanes_below(mm);
+        if (one && pos < R) g[pos] = id[t];
+        w += __popcll(mm);
+    }
+    const uint32_t g0 = seq[0];
+    for (uint32_t j = w + lane; j < R; j += 64u) g[j] = g0;
+}
+
 }  // namespace
+
+hipError_t launch_rev_edges(const RevArgs& a, hipStream_t st) {
+    if (!a.n) return hipSuccess;
+    if (a.I < 1 || a.I > 64 || a.R < 1 || a.R > a.I) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_zero_u32, dim3((a.n + 255) / 256), dim3(256), 0, st, a.cnt, a.n);
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, st, reinterpret_cast<uint32_t*>(a.used), 2u);
+    hipLaunchKernelGGL(k_rev_count, dim3((a.n + 255) / 256), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_rev_start, dim3((a.n + 1023) / 1024), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(k_rev_fill, dim3((a.n + 255) / 256), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_rev_merge, dim3(a.n), dim3(64), 0, st, a);
+    return hipGetLastError();
+}
 
 hipError_t launch_prune(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t* offset, uint32_t P,
                         uint32_t* out, hipStream_t st) {
     if (!N) return hipSuccess;
     if (I < 1 || I > 64) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_prune, dim3(N), dim3(64), size_t(I) * I * sizeof(uint32_t), st, knn, N, I, offset, P, out);
+    hipLaunchKernelGGL(k_prune, dim3(N), dim3(64), 0, st, knn, N, I, offset, P, out);
     return hipGetLastError();
 }
 
