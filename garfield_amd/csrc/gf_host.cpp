@@ -404,10 +404,11 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
         }
         build_subcells(h, gidx, size, ix);
         // Integer-valued data in [0, 255]: int8 tiles of the MFMA brute force.
-        bool ints = ix.sub && !gf::half_rows(ix.vdtype) && ix.vdtype != GF_VEC_I8Q && D % 64 == 0 && D <= 256;
+        bool ints = ix.sub && !gf::half_rows(ix.vdtype) && ix.vdtype != GF_VEC_I8Q && D <= 256;
         for (size_t i = 0; ints && i < v.size(); ++i) ints = v[i] >= 0.0f && v[i] <= 255.0f && v[i] == std::floor(v[i]);
         if (ints) {
-            ix.trec.alloc(size_t(ix.ntile) * gf::bf_rec_bytes(D, ix.AW));
+            ix.Db = gf::bf_i8_dim(D);
+            ix.trec.alloc(size_t(ix.ntile) * gf::bf_rec_bytes(ix.Db, ix.AW));
             GF_HIP(gf::launch_tile_rec(vec_f32_dev, false, D, ix.tmeta.p, ix.AW, ix.ntile, ix.trec.p,
                                       ix.stream));
             ix.i8 = true;
@@ -441,9 +442,10 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
             }
             // the brute force's tile records: its tiles' rows in MFMA operand
             // order, contiguous per tile, with their meta records and norms
-            const uint32_t KS = fvt == 1 ? D / 32 : D / 16;
+            ix.Db = gf::bf_float_dim(fvt, D);
+            const uint32_t KS = fvt == 1 ? ix.Db / 32 : ix.Db / 16;
             ix.frec.alloc(size_t(ix.ntile) * gf::bf_frec_bytes(KS, ix.AW));
-            GF_HIP(gf::launch_tile_frec(ix.vec.p, fvt, D, ix.tmeta.p, ix.xnormf.p, ix.AW, ix.ntile, ix.frec.p,
+            GF_HIP(gf::launch_tile_frec(ix.vec.p, fvt, D, ix.Db, ix.tmeta.p, ix.xnormf.p, ix.AW, ix.ntile, ix.frec.p,
                                         ix.stream));
             ix.hf = true;
             // Binary16 rows' first pass (a launch of its own): one in four
@@ -829,7 +831,7 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             // products.
             const uint32_t D = ix->D;
             const bool h = ix->vdtype == GF_VEC_F16;
-            const double u = std::ldexp(1.0, -24), gam = (D + 2) * u / (1.0 - (D + 2) * u);
+            const double u = std::ldexp(1.0, -24), gam = (ix->Db + 2) * u / (1.0 - (ix->Db + 2) * u);
             std::vector<float> eps(Q), qn(h ? 0 : Q);
             for (uint32_t q = 0; q < Q; ++q) {
                 double s = 0.0;
@@ -851,6 +853,15 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
                 b->qnf.upload(qn);
             }
             b->heps.upload(eps);
+            if (ix->Db != D) {
+                // the kernel's queries, zero padded to the records' dimension
+                const size_t es = h ? 2 : 4;
+                b->qpad.alloc(size_t(Q) * ix->Db * es);
+                GF_HIP(hipMemsetAsync(b->qpad.p, 0, b->qpad.n, ix->stream));
+                GF_HIP(hipMemcpy2DAsync(b->qpad.p, ix->Db * es,
+                                        h ? static_cast<const void*>(b->q16v.p) : static_cast<const void*>(b->qf32.p),
+                                        D * es, D * es, Q, hipMemcpyDeviceToDevice, ix->stream));
+            }
         }
         if (ix->vdtype == GF_VEC_I8Q) {
             // rows [c | s]: c_d = fma(s_d, z_d, alpha q_d), the query less
@@ -877,9 +888,9 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             for (size_t i = 0; ints && i < nq; ++i)
                 ints = queries[i] >= 0.0f && queries[i] <= 255.0f && queries[i] == std::floor(queries[i]);
             if (ints) {
-                b->q8.alloc(nq);
+                b->q8.alloc(size_t(Q) * ix->Db);
                 b->nq.alloc(Q);
-                GF_HIP(gf::launch_q_i8(b->qf32.p, Q, ix->D, b->q8.p, b->nq.p, ix->stream));
+                GF_HIP(gf::launch_q_i8(b->qf32.p, Q, ix->D, ix->Db, b->q8.p, b->nq.p, ix->stream));
                 b->i8 = true;
             }
         }
@@ -1143,11 +1154,22 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     // Brute-force route on MFMA when vectors and queries are int8-exact:
     // work items of (sub-cell, <= 64 queries whose range reaches it),
     // scheduled on the device.
-    const bool gemm = ix->i8 && b->i8 && K <= gf::kBfKMax;
+    // Dimensions that run padded (Db > D) take it for larger batches only:
+    // below these lines the gather kernel's parts finish before the MFMA
+    // route's chain of launches would.  rows x (row bytes + 160) is the
+    // gather's cost if every row passes; measured at 100 dimensions, all rows
+    // passing / 1 to 50 % passing, gather against MFMA: int8 3.2M rows (1.8
+    // GB) 199 / 130 us against 264 / 268, 6M rows 399 / 181 against 234 /
+    // 220; fp32 6M rows (3.4 GB) 398 / 179 against 384 / 326, 12M rows 711 /
+    // 242 against 417 / 342.
+    const double gather_bytes = double(Q) * ix->N * (ix->rowbytes + 160.0);
+    const bool padded = ix->Db != ix->D;
+    const bool gemm = ix->i8 && b->i8 && K <= gf::kBfKMax && !(padded && gather_bytes < 1.8e9);
     // Binary16 rows: the same items on fp16 MFMA, candidates within the
     // distances' error bound re-ranked exactly (k_bf_f16, k_bf_f16_final).
     const int fvt = ix->vdtype == GF_VEC_F16 ? 1 : 0;
-    const bool gemm_h = !gemm && ix->hf && b->qnf.n == Q && gf::bf_float_supported(fvt, ix->D, ix->AW, K);
+    const bool gemm_h = !gemm && ix->hf && b->qnf.n == Q && gf::bf_float_supported(fvt, ix->D, ix->AW, K) &&
+                        !(padded && gather_bytes < 3.4e9);
     const bool sched_bf = gemm || gemm_h;
     const uint32_t KP = gemm_h ? gf::kBfHKT : K;   // keys per (query, item) in the partial area
     const uint32_t seed_tiles = gemm_h ? gf::kBfHSeedTiles : gf::kBfSeedTiles;
@@ -1254,13 +1276,15 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             gf::BfHArgs ha{};
             ha.sa = sub_args(*ix);
             ha.rec = ix->frec.p;
-            ha.q16 = fvt == 1 ? static_cast<const void*>(b->q16v.p) : static_cast<const void*>(b->qf32.p);
+            ha.q16 = b->qpad.p ? static_cast<const void*>(b->qpad.p)
+                     : fvt == 1 ? static_cast<const void*>(b->q16v.p)
+                                : static_cast<const void*>(b->qf32.p);
             ha.qnorm = b->qnf.p; ha.eps = b->heps.p; ha.lo = b->lo.p; ha.hi = b->hi.p;
             ha.items = b->items.p; ha.nitems = tot + 4; ha.bq = b->bq.p; ha.part_off = b->part_off.p;
             ha.pcnt = b->pcnt.p; ha.part = b->part.p; ha.gbound = b->gbound.p; ha.over = b->hover.p;
             ha.ok = tot + 3;
             if (seeds) { ha.sitems = b->sitems.p; ha.nseed = tot + 5; ha.nseed_cap = scap; ha.seeds_on = 1; }
-            ha.K = K; ha.D = ix->D;
+            ha.K = K; ha.D = ix->Db;
             GF_HIP(gf::launch_stamp(stamp + 3, st));
             // Binary16 rows: the seeds alone, then (two passes) the
             // first-pass sub-cells' items, then the rest, each launch
@@ -1298,7 +1322,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         ga.part_off = b->part_off.p; ga.part = b->part.p; ga.gbound = b->gbound.p;
         ga.ok = tot + 3;
         if (seeds) { ga.sitems = b->sitems.p; ga.nseed = tot + 5; ga.nseed_cap = scap; ga.seeds_on = 1; }
-        ga.K = K; ga.D = ix->D;
+        ga.K = K; ga.D = ix->Db;
         gf::BfFinalArgs fa{};
         fa.gbound = b->gbound.p; fa.bfq = b->sched.p; fa.srange = tot + 14; fa.part_off = b->part_off.p; fa.pcnt = b->pcnt.p;
         fa.ok = tot + 3; fa.part = b->part.p; fa.counts = b->counts.p; fa.cells = b->cells.p;
@@ -1507,7 +1531,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // Item schedule: every (query, sub-cell) pair costs 2 D ops per
             // point; every item streams its sub-cell's tiles once; the final
             // merge reads the appended keys.
-            const double tile_bytes = (ix->D / 64) * 1024.0 + 32 * 4.0 + 16.0 * (1 + ix->AW) * 4.0;
+            const double tile_bytes = (ix->Db / 64) * 1024.0 + 32 * 4.0 + 16.0 * (1 + ix->AW) * 4.0;
             stats->ops_bruteforce = 2.0 * ix->D * double(sm[9]);
             stats->bytes_bruteforce = double(sm[10]) * tile_bytes + double(dt[9]) * K * 16.0;
             stats->bf_mfma = 1;
@@ -1515,7 +1539,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // fp16 items: every (query, sub-cell) pair costs 2 D flops per
             // point; every item streams its sub-cell's rows and meta; the
             // final re-rank gathers the candidates' rows
-            const double tile_bytes = 16.0 * ix->D * 2.0 + 16.0 * (2 + ix->AW) * 4.0;
+            const double tile_bytes = 16.0 * ix->Db * 2.0 + 16.0 * (2 + ix->AW) * 4.0;
             stats->ops_bruteforce = 2.0 * ix->D * double(sm[9]);
             stats->bytes_bruteforce = double(sm[10]) * tile_bytes + b_dist * ix->rowbytes + double(dt[9]) * K * 16.0;
             stats->bf_mfma = 2;

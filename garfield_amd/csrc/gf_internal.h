@@ -168,7 +168,7 @@ __host__ __device__ inline uint32_t bf_frec_bytes(uint32_t KS, uint32_t AW) { re
 struct BfGemmArgs {
     SubArgs sa;
     const uint8_t* rec;        // tile records (bf_rec_bytes each)
-    const int8_t* q8;          // Q*D queries shifted by -128
+    const int8_t* q8;          // Q*D queries shifted by -128 (D: bf_i8_dim)
     const int32_t* nq;         // |q - 128|^2
     const float* lo;
     const float* hi;
@@ -201,7 +201,7 @@ constexpr uint32_t kBfHKT = 32;       // keys an item keeps per query
 struct BfHArgs {
     SubArgs sa;
     const uint8_t* rec;        // tile records (bf_frec_bytes each)
-    const void* q16;           // Q*D queries of the rows' type
+    const void* q16;           // Q*D queries of the rows' type (D: bf_float_dim)
     const float* qnorm;        // per query |q|^2
     const float* eps;          // per query bound of |d' - d|
     const float* lo;
@@ -235,9 +235,17 @@ struct BfHFinal {
     const float* eps;
     const uint32_t* selcount;
 };
-// vt 1 (binary16 rows): D in {64, 96, 128, 256, 512, 768}; vt 0 (fp32
-// rows): D in {64, 96, 128, 256}; AW 1 or 2; K <= 10.
+// The dimension that the MFMA brute force of D-dimensional float rows runs
+// at: D with zeros up to the next of 64, 96, 128, 256, 512, 768 (vt 1,
+// binary16 rows, D >= 64) or 64, 96, 128, 256 (vt 0, fp32 rows, D >= 64);
+// 0: not supported.  Zeros add nothing to norms or products.  Against the
+// gather kernel, 100 dimensions at 128, 150k points, 777 queries: 1.36 ->
+// 0.39 ms (fp32 rows); integer rows (bf_i8_dim) 1.48 -> 0.27 ms.
+uint32_t bf_float_dim(int vt, uint32_t D);
+// bf_float_dim, AW 1 or 2, K <= 10.
 bool bf_float_supported(int vt, uint32_t D, uint32_t AW, uint32_t K);
+// The dimension that the int8 MFMA brute force runs at (D <= 256).
+inline uint32_t bf_i8_dim(uint32_t D) { return (D + 63u) / 64u * 64u; }
 hipError_t launch_bf_float(const BfHArgs& a, int vt, uint32_t AW, uint32_t ncu, hipStream_t st);
 // Brute-force queries of the schedule range srange in a.sched (binary16 or fp32 rows).
 hipError_t launch_bf_f16_final(const RowShape& rs, const TravArgs& a, const BfHFinal& f, uint32_t grid,
@@ -486,8 +494,9 @@ hipError_t launch_tile_i8(const void* vec_cm, bool u8, uint32_t D, const uint32_
                           int8_t* vt, int32_t* tnorm, hipStream_t st);
 // The brute force's tile records (bf_rec_bytes each) from the same inputs.
 // Float tile records (bf_frec_bytes) of ntile tiles from cell-major rows of
-// type vt (1 binary16, 0 fp32) and their norms.
-hipError_t launch_tile_frec(const void* vec, int vt, uint32_t D, const uint32_t* tmeta, const float* xnorm,
+// type vt (1 binary16, 0 fp32; D dimensions, Dp = bf_float_dim in the
+// records) and their norms.
+hipError_t launch_tile_frec(const void* vec, int vt, uint32_t D, uint32_t Dp, const uint32_t* tmeta, const float* xnorm,
                             uint32_t AW, uint32_t ntile, uint8_t* rec, hipStream_t st);
 hipError_t launch_tile_rec(const void* vec_cm, bool u8, uint32_t D, const uint32_t* tmeta, uint32_t AW, uint32_t ntile,
                            uint8_t* rec, hipStream_t st);
@@ -508,7 +517,7 @@ hipError_t launch_sched(const SchedArgs& a, hipStream_t st);
 hipError_t launch_stats(const StatsArgs& a, hipStream_t st);
 hipError_t launch_total(const uint32_t* cnt, const uint32_t* start, uint32_t n, uint32_t cap, uint32_t mul,
                         uint64_t cap2, uint32_t* out, hipStream_t st);
-hipError_t launch_q_i8(const float* q, uint32_t Q, uint32_t D, int8_t* q8, int32_t* nq, hipStream_t st);
+hipError_t launch_q_i8(const float* q, uint32_t Q, uint32_t D, uint32_t Dp, int8_t* q8, int32_t* nq, hipStream_t st);
 hipError_t launch_f2h(const float* x, uint16_t* out, size_t n, float alpha, hipStream_t st);
 hipError_t launch_f2h_pad(const float* x, uint32_t rows, uint32_t D, uint16_t* out,
                           uint32_t rows_pad, uint32_t Dp, float alpha, hipStream_t st);

@@ -3923,20 +3923,23 @@ __device__ void bf_float_items(const BfHArgs& p) {
 // Float tile records (bf_frec_bytes) for the float MFMA brute force: one
 // wave per tile copies its 16 rows' operand chunks into MFMA operand order
 // (BfChunk<VT>::at), then the meta record and the rows' norms; an empty slot
-// (row kEmpty) gets zero operands and norm.
+// (row kEmpty) and the dimensions from D to Dp get zero operands.
 template <int VT>
-__global__ __launch_bounds__(64) void k_tile_frec(const void* vec, uint32_t D, const uint32_t* tmeta,
+__global__ __launch_bounds__(64) void k_tile_frec(const void* vec, uint32_t D, uint32_t Dp, const uint32_t* tmeta,
                                                   const float* xnorm, uint32_t AW, uint8_t* rec) {
     typedef BfChunk<VT> CH;
     typedef typename CH::E ElemT;
     const uint32_t t = blockIdx.x, lane = lane_id();
-    const uint32_t KS = VT == 1 ? D / 32u : D / 16u, MW = 16u * (1u + AW);
+    const uint32_t KS = VT == 1 ? Dp / 32u : Dp / 16u, MW = 16u * (1u + AW);
     uint8_t* dst = rec + size_t(t) * bf_frec_bytes(KS, AW);
     const uint32_t row = tmeta[size_t(t) * MW + (lane & 15u)];
     const ElemT* src = reinterpret_cast<const ElemT*>(vec) + size_t(row == kEmpty ? 0u : row) * D;
     for (uint32_t k = 0; k < KS; ++k) {
         uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (row != kEmpty) v = *reinterpret_cast<const uint4*>(CH::at(src, D, lane >> 4, int(k)));
+        // a 16-byte chunk lies inside the row or in its zero padding: D is a
+        // multiple of the chunk's elements
+        const ElemT* at = CH::at(src, Dp, lane >> 4, int(k));
+        if (row != kEmpty && uint32_t(at - src) < D) v = *reinterpret_cast<const uint4*>(at);
         *reinterpret_cast<uint4*>(dst + k * 1024u + lane * 16u) = v;
     }
     uint32_t* tail = reinterpret_cast<uint32_t*>(dst + KS * 1024u);
@@ -4122,17 +4125,17 @@ __global__ __launch_bounds__(64) void k_bf_final(BfFinalArgs p) {
 // tile order and per tile [-floor(|x'|^2 / 2) x 16][|x'|^2 x 16] (padding
 // points are all zero).
 template <typename T>
-__global__ __launch_bounds__(64) void k_tile_i8(const T* vec, uint32_t D, const uint32_t* tmeta, uint32_t AW,
-                                               int8_t* vt, size_t vstride, int32_t* tnorm, size_t nstride,
+__global__ __launch_bounds__(64) void k_tile_i8(const T* vec, uint32_t D, uint32_t KS, const uint32_t* tmeta,
+                                               uint32_t AW, int8_t* vt, size_t vstride, int32_t* tnorm, size_t nstride,
                                                uint32_t* mdst, size_t mstride) {
-    // Tile t's k-steps at vt + t vstride, its norms at tnorm + t nstride and,
+    // Tile t's KS k-steps (dimensions beyond D are 0 after the shift) at
+    // vt + t vstride, its norms at tnorm + t nstride and,
     // with mdst, a copy of its meta (16 (1 + AW) words) at mdst + t mstride.
     const uint32_t t = blockIdx.x, lane = lane_id();
     const uint32_t col = lane & 15u;
     const uint32_t MW = 16u * (1u + AW);
     const uint32_t row = tmeta[size_t(t) * MW + col];
     const bool valid = row != 0xFFFFFFFFu;
-    const uint32_t KS = D / 64u;
     if (mdst && lane < MW) mdst[size_t(t) * mstride + lane] = tmeta[size_t(t) * MW + lane];
     if constexpr (sizeof(T) == 1) {
         // u8 rows: each lane moves its 16 bytes of a k-step with one load and
@@ -4141,7 +4144,8 @@ __global__ __launch_bounds__(64) void k_tile_i8(const T* vec, uint32_t D, const 
         int32_t n = 0;
         for (uint32_t s = 0; s < KS; ++s) {
             uint4 v = make_uint4(0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u);
-            if (valid) v = *reinterpret_cast<const uint4*>(vec + size_t(row) * D + s * 64u + (lane >> 4) * 16u);
+            const uint32_t k0 = s * 64u + (lane >> 4) * 16u;   // u8 rows: D is a multiple of 16
+            if (valid && k0 < D) v = *reinterpret_cast<const uint4*>(vec + size_t(row) * D + k0);
             v.x ^= 0x80808080u; v.y ^= 0x80808080u; v.z ^= 0x80808080u; v.w ^= 0x80808080u;
             *reinterpret_cast<uint4*>(vt + size_t(t) * vstride + s * 1024u + lane * 16u) = v;
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -4165,7 +4169,7 @@ __global__ __launch_bounds__(64) void k_tile_i8(const T* vec, uint32_t D, const 
         int8_t* dst = vt + size_t(t) * vstride + s * 1024u + lane * 16u;
         for (uint32_t j = 0; j < 16; ++j) {
             const uint32_t k = s * 64u + (lane >> 4) * 16u + j;
-            dst[j] = valid ? int8_t(int32_t(vec[size_t(row) * D + k]) - 128) : int8_t(0);
+            dst[j] = valid && k < D ? int8_t(int32_t(vec[size_t(row) * D + k]) - 128) : int8_t(0);
         }
     }
     if (lane < 16) {
@@ -4180,12 +4184,12 @@ __global__ __launch_bounds__(64) void k_tile_i8(const T* vec, uint32_t D, const 
     }
 }
 
-__global__ __launch_bounds__(64) void k_q_i8(const float* q, uint32_t D, int8_t* q8, int32_t* nq) {
+__global__ __launch_bounds__(64) void k_q_i8(const float* q, uint32_t D, uint32_t Dp, int8_t* q8, int32_t* nq) {
     const uint32_t r = blockIdx.x, lane = lane_id();
     int32_t n = 0;
-    for (uint32_t k = lane; k < D; k += 64u) {
-        const int32_t v = int32_t(q[size_t(r) * D + k]) - 128;
-        q8[size_t(r) * D + k] = int8_t(v);
+    for (uint32_t k = lane; k < Dp; k += 64u) {
+        const int32_t v = k < D ? int32_t(q[size_t(r) * D + k]) - 128 : 0;
+        q8[size_t(r) * Dp + k] = int8_t(v);
         n += v * v;
     }
 #pragma unroll
@@ -4886,21 +4890,20 @@ hipError_t launch_bf_f16_final_t(const TravArgs& a, const BfHFinal& f, uint32_t 
 }
 }  // namespace
 
+uint32_t bf_float_dim(int vt, uint32_t D) {
+    if (D < 64) return 0;
+    static constexpr uint32_t dims[] = {64, 96, 128, 256, 512, 768};
+    for (uint32_t d : dims)
+        if (D <= d) return (vt == 1 || (vt == 0 && d <= 256)) ? d : 0;
+    return 0;
+}
+
 bool bf_float_supported(int vt, uint32_t D, uint32_t AW, uint32_t K) {
-    if (!(AW == 1 || AW == 2) || K < 1 || K > 10) return false;
-    if (vt == 1) {
-        const uint32_t ks = D / 32;
-        return D % 32 == 0 && (ks == 2 || ks == 3 || ks == 4 || ks == 8 || ks == 16 || ks == 24);
-    }
-    if (vt == 0) {
-        const uint32_t ks = D / 16;
-        return D % 16 == 0 && (ks == 4 || ks == 6 || ks == 8 || ks == 16);
-    }
-    return false;
+    return (AW == 1 || AW == 2) && K >= 1 && K <= 10 && bf_float_dim(vt, D) != 0;
 }
 
 hipError_t launch_bf_float(const BfHArgs& a, int vt, uint32_t AW, uint32_t ncu, hipStream_t st) {
-    if (!bf_float_supported(vt, a.D, AW, a.K) || ncu == 0) return hipErrorInvalidValue;
+    if (!bf_float_supported(vt, a.D, AW, a.K) || bf_float_dim(vt, a.D) != a.D || ncu == 0) return hipErrorInvalidValue;
 #define BFH(VT_, KS_)                                                                        \
     case KS_:                                                                                \
         return AW == 1 ? launch_bf_float_t<VT_, KS_, 1>(a, ncu, st) : launch_bf_float_t<VT_, KS_, 2>(a, ncu, st);
@@ -5060,36 +5063,37 @@ hipError_t launch_tile_i8(const void* vec_cm, bool u8, uint32_t D, const uint32_
     const size_t vs = size_t(D / 64) * 1024u;
     if (u8)
         hipLaunchKernelGGL(k_tile_i8<uint8_t>, dim3(ntile), dim3(64), 0, st, static_cast<const uint8_t*>(vec_cm), D,
-                           tmeta, AW, vt, vs, tnorm, size_t(32), static_cast<uint32_t*>(nullptr), size_t(0));
+                           D / 64u, tmeta, AW, vt, vs, tnorm, size_t(32), static_cast<uint32_t*>(nullptr), size_t(0));
     else
         hipLaunchKernelGGL(k_tile_i8<float>, dim3(ntile), dim3(64), 0, st, static_cast<const float*>(vec_cm), D,
-                           tmeta, AW, vt, vs, tnorm, size_t(32), static_cast<uint32_t*>(nullptr), size_t(0));
+                           D / 64u, tmeta, AW, vt, vs, tnorm, size_t(32), static_cast<uint32_t*>(nullptr), size_t(0));
     return hipGetLastError();
 }
 
-hipError_t launch_tile_frec(const void* vec, int vt, uint32_t D, const uint32_t* tmeta, const float* xnorm,
+hipError_t launch_tile_frec(const void* vec, int vt, uint32_t D, uint32_t Dp, const uint32_t* tmeta, const float* xnorm,
                             uint32_t AW, uint32_t ntile, uint8_t* rec, hipStream_t st) {
     if (!ntile) return hipSuccess;
     if (vt == 1)
-        hipLaunchKernelGGL(k_tile_frec<1>, dim3(ntile), dim3(64), 0, st, vec, D, tmeta, xnorm, AW, rec);
+        hipLaunchKernelGGL(k_tile_frec<1>, dim3(ntile), dim3(64), 0, st, vec, D, Dp, tmeta, xnorm, AW, rec);
     else
-        hipLaunchKernelGGL(k_tile_frec<0>, dim3(ntile), dim3(64), 0, st, vec, D, tmeta, xnorm, AW, rec);
+        hipLaunchKernelGGL(k_tile_frec<0>, dim3(ntile), dim3(64), 0, st, vec, D, Dp, tmeta, xnorm, AW, rec);
     return hipGetLastError();
 }
 
 hipError_t launch_tile_rec(const void* vec_cm, bool u8, uint32_t D, const uint32_t* tmeta, uint32_t AW, uint32_t ntile,
                            uint8_t* rec, hipStream_t st) {
     if (!ntile) return hipSuccess;
-    const size_t rb = bf_rec_bytes(D, AW), ks = size_t(D / 64) * 1024u;
+    const uint32_t Dp = bf_i8_dim(D);
+    const size_t rb = bf_rec_bytes(Dp, AW), ks = size_t(Dp / 64) * 1024u;
     int8_t* vt = reinterpret_cast<int8_t*>(rec);
     int32_t* tn = reinterpret_cast<int32_t*>(rec + ks);
     uint32_t* md = reinterpret_cast<uint32_t*>(rec + ks + 128u);
     if (u8)
         hipLaunchKernelGGL(k_tile_i8<uint8_t>, dim3(ntile), dim3(64), 0, st, static_cast<const uint8_t*>(vec_cm), D,
-                           tmeta, AW, vt, rb, tn, rb / 4u, md, rb / 4u);
+                           Dp / 64u, tmeta, AW, vt, rb, tn, rb / 4u, md, rb / 4u);
     else
         hipLaunchKernelGGL(k_tile_i8<float>, dim3(ntile), dim3(64), 0, st, static_cast<const float*>(vec_cm), D,
-                           tmeta, AW, vt, rb, tn, rb / 4u, md, rb / 4u);
+                           Dp / 64u, tmeta, AW, vt, rb, tn, rb / 4u, md, rb / 4u);
     return hipGetLastError();
 }
 
@@ -5139,9 +5143,9 @@ hipError_t launch_total(const uint32_t* cnt, const uint32_t* start, uint32_t n, 
     return hipGetLastError();
 }
 
-hipError_t launch_q_i8(const float* q, uint32_t Q, uint32_t D, int8_t* q8, int32_t* nq, hipStream_t st) {
+hipError_t launch_q_i8(const float* q, uint32_t Q, uint32_t D, uint32_t Dp, int8_t* q8, int32_t* nq, hipStream_t st) {
     if (!Q) return hipSuccess;
-    hipLaunchKernelGGL(k_q_i8, dim3(Q), dim3(64), 0, st, q, D, q8, nq);
+    hipLaunchKernelGGL(k_q_i8, dim3(Q), dim3(64), 0, st, q, D, Dp, q8, nq);
     return hipGetLastError();
 }
 
