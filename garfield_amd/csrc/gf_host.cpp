@@ -1174,6 +1174,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     const uint32_t KP = gemm_h ? gf::kBfHKT : K;   // keys per (query, item) in the partial area
     const uint32_t seed_tiles = gemm_h ? gf::kBfHSeedTiles : gf::kBfSeedTiles;
     const uint32_t NS = ix->NS;
+    const uint32_t tch = gemm_h ? gf::kBfHItemTiles : gf::bf_item_tiles(NS, Q);   // tiles per item, at most
     b->pass_pending = sched_bf && !b->sel_exact;
     if (sched_bf) {
         if (!b->bcnt.n) {
@@ -1182,7 +1183,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         }
         // item slots: a sub-cell adds up to two partial query blocks per
         // tile chunk beyond pairs / 64
-        const size_t islots = size_t(NS) + ix->ntile / gf::kBfMaxItemTiles + 1;
+        const size_t islots = size_t(NS) + ix->ntile / tch + 1;
         if (!b->part.n) b->alloc_pairs(size_t(Q) * 64, KP, Q, NS, islots);
         if (b->rq.n < Q) {
             b->rq.alloc(Q); b->rseed.alloc(Q);
@@ -1227,7 +1228,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         sc.bstart = b->bstart.p; sc.bq = b->bq.p; sc.qcap = b->qcap;
         sc.ok = tot + 3; sc.nbf = tot + 9;
         sc.qlist = b->sched.p; sc.qrange = tot + 14;   // the brute-force queries of the schedule
-        sc.tch = gf::kBfMaxItemTiles;
+        sc.tch = tch;
         if (!b->bf_all) {
             GF_HIP(gf::launch_cell_flags(Q, ix->P, b->cells.p, b->counts.p, b->little.p, b->bfmask.p, st));
             sc.bfm = b->bfmask.p;
@@ -1243,7 +1244,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             sd.sa = sc.sa; sd.Q = Q; sd.postfilter = sc.postfilter; sd.counts = sc.counts; sd.little = sc.little;
             sd.cells = b->cells.p; sd.lo = sc.lo; sd.hi = sc.hi; sd.bfm = sc.bfm; sd.bP = sc.bP;
             sd.qlist = sc.qlist; sd.qrange = sc.qrange; sd.qcap = b->qcap; sd.tch = seed_tiles;
-            sd.itch = gf::kBfMaxItemTiles;
+            sd.itch = tch;
             sd.scnt = b->scnt.p; sd.bq = b->bq.p; sd.nsub = b->nsub.p;
             sd.rq = b->rq.p; sd.rseed = b->rseed.p; sd.rlo = b->rlo.p; sd.rhi = b->rhi.p;
             GF_HIP(gf::launch_bfseed(sd, Q, st));
@@ -1262,12 +1263,12 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         // of the items under those bounds.  Both k_bfitems launches take
         // the sub-cells in the same order (counts, scan, fill).
         const bool two = ix->sorder.n == NS && ix->ns1 > 0 && ix->ns1 < NS;
-        GF_HIP(gf::launch_bfitems(b->bcnt.p, b->bin.p, b->bstart.p, b->qcap, ix->stile.p, gf::kBfMaxItemTiles, NS, b->icnt.p, b->ioff.p,
+        GF_HIP(gf::launch_bfitems(b->bcnt.p, b->bin.p, b->bstart.p, b->qcap, ix->stile.p, tch, NS, b->icnt.p, b->ioff.p,
                                   b->items.p, tot + 4, tot + 3, false, st, nullptr, nullptr, nullptr, 0,
                                   two ? ix->sorder.p : nullptr, two ? ix->ns1 : 0u, nullptr));
         GF_HIP(gf::launch_scan_small(b->icnt.p, NS, b->ioff.p, st));
         const uint32_t scap = uint32_t(b->sitems.n);
-        GF_HIP(gf::launch_bfitems(b->bcnt.p, b->bin.p, b->bstart.p, b->qcap, ix->stile.p, gf::kBfMaxItemTiles, NS, b->icnt.p, b->ioff.p,
+        GF_HIP(gf::launch_bfitems(b->bcnt.p, b->bin.p, b->bstart.p, b->qcap, ix->stile.p, tch, NS, b->icnt.p, b->ioff.p,
                                   b->items.p, tot + 4, tot + 3, true, st, seeds ? b->scnt.p : nullptr,
                                   b->sitems.p, tot + 5, scap, two ? ix->sorder.p : nullptr, two ? ix->ns1 : 0u,
                                   two ? tot + 6 : nullptr, seed_tiles));
@@ -1487,7 +1488,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     const uint32_t* dt = b->h_tot.p;
     if (sched_bf && !dt[3]) {
         // the pair lists outgrew their buffers: grow them and run the brute force again
-        b->alloc_pairs(size_t(dt[2]) + dt[2] / 4 + 1024, KP, Q, NS, size_t(NS) + ix->ntile / gf::kBfMaxItemTiles + 1);
+        b->alloc_pairs(size_t(dt[2]) + dt[2] / 4 + 1024, KP, Q, NS, size_t(NS) + ix->ntile / tch + 1);
         GF_HIP(gf::launch_stamp(stamp + 1, st));
         launch_gemm(false);
         enqueue_tail();

@@ -151,6 +151,22 @@ constexpr uint32_t kBfTile = 16;      // points per tile
 constexpr uint32_t kBfKMax = 16;      // largest K of the MFMA route
 constexpr uint32_t kBfQB = 64;        // queries per work item
 constexpr uint32_t kBfMaxItemTiles = 65536;   // tiles per MFMA work item (keeps buffer offsets below 2^31)
+// Tiles per item of the int8 route: a sub-cell whole while there are many
+// items per wave, else even chunks, so that the last items of a launch are
+// short and a small batch has items for every wave.  By the most items there
+// can be: 160k (1M points, 10k queries) 731 us a search whole, 737 at 48 and
+// 739 at 32; 33k (1M, 2000) 376 whole, 351 at 32, 358 at 16; 16k (250k, 4000)
+// 387 whole, 352 at 32, 334 at 16; 2k (60k, 2000) 362, 298, 266.
+inline uint32_t bf_item_tiles(uint32_t NS, uint32_t Q) {
+    const uint64_t most = uint64_t(NS) * ((Q + 63u) / 64u);
+    return most <= 20000u ? 16u : most <= 65536u ? 32u : kBfMaxItemTiles;
+}
+// The same for the float route, whose items are longer (a workgroup each, a
+// tile record a step): 48 at all sizes.  Whole sub-cells against 48 (even
+// chunks, so 25 to 48): 96-d fp32, 300k points, 3001 queries 1263 -> 951 us,
+// 1M points, 10k queries 7.32 -> 5.68 ms; 768-d binary16, 120k points, 4096
+// queries 914 -> 733 us, 400k points, 10k queries 2.38 -> 2.42 ms.
+constexpr uint32_t kBfHItemTiles = 48;
 constexpr uint32_t kBfSeedTiles = 16;         // tiles per seed item: a seed sub-cell spreads over several waves
 constexpr uint32_t kBfHFirstPass = 4;         // binary16 rows' first pass: sub-cells with grid hash % 4 == 0
 constexpr uint32_t kBfHSeedTiles = 128;       // the same for the float MFMA route (measured: C4 5.6 ms at 128, 6.0 at 16)

@@ -2834,6 +2834,9 @@ __device__ __forceinline__ uint32_t tile_chunks(const uint32_t* stile, uint32_t 
     const uint32_t nt = stile[s + 1] - stile[s];
     return tch ? (nt + tch - 1) / tch : 1u;
 }
+// Tiles per chunk of nt tiles in nc chunks: even ones, no more than the tch
+// that gave nc (48 tiles and a rest of 6 cost an item what 27 and 27 do not).
+__device__ __forceinline__ uint32_t chunk_tiles(uint32_t nt, uint32_t nc) { return nc ? (nt + nc - 1u) / nc : 0u; }
 
 // Seed choice, one wave per candidate query (see BfSeedArgs): among the
 // sub-cells of the first cell of the query's list that its brute force
@@ -3239,7 +3242,7 @@ __global__ __launch_bounds__(256) void k_bfitems(const uint32_t* bcnt, const uin
         // seed items go to their own list (order is free: each is one
         // sub-cell), in chunks of stch tiles, one wave per item (no padding)
         const uint32_t nc = tile_chunks(stile, s, stch), gs = (ns + kBfQB - 1) / kBfQB;
-        const uint32_t t0 = stile[s], t1 = stile[s + 1], step = stch ? stch : (t1 - t0);
+        const uint32_t t0 = stile[s], t1 = stile[s + 1], step = chunk_tiles(t1 - t0, nc);
         uint32_t k0 = 0;
         if (lane == 0) k0 = atomicAdd(nseed, gs * nc);
         k0 = uint32_t(__shfl(int(k0), 0, 64));
@@ -3259,7 +3262,7 @@ __global__ __launch_bounds__(256) void k_bfitems(const uint32_t* bcnt, const uin
         if (lane == 0) icnt[ks] = g * nc;
         return;
     }
-    const uint32_t t0 = stile[s], t1 = stile[s + 1], step = tch ? tch : (t1 - t0);
+    const uint32_t t0 = stile[s], t1 = stile[s + 1], step = chunk_tiles(t1 - t0, nc);
     const uint32_t k0 = ioff[ks];
     if (lane == 0 && nitems_a) {
         if (ks + 1 == ns1) *nitems_a = k0 + g * nc;
