@@ -1436,7 +1436,22 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // cell: no traversal is launched)
             gf::TravArgs at = a;
             at.srange = tot + 12;
-            if (channels == 2) GF_HIP(gf::launch_traverse_dual(ix->rs, at, lds, Q, st));
+            if (channels == 2) {
+                // only the device knows how many queries are traversed: the
+                // launch whose range does not hold their number ends at once
+                const gf::VisitedRows vr = gf::visited_rows(ix->N, Lpad, uint32_t(ix->ncu));
+                if (vr.bits) {
+                    gf::TravArgs ar = at;
+                    ar.hsize = vr.words;
+                    ar.vbits = vr.bits;
+                    ar.qmax = vr.most;
+                    GF_HIP(gf::launch_traverse_dual(ix->rs, ar, gf::trav_dual_lds_bytes(Lpad, vr.words),
+                                                    std::min(Q, vr.most), st));
+                }
+                at.qmin = vr.bits ? vr.most + 1 : 0u;
+                at.qmax = Q;
+                if (at.qmin <= Q) GF_HIP(gf::launch_traverse_dual(ix->rs, at, lds, Q, st));
+            }
             else GF_HIP(gf::launch_traverse(ix->rs, at, lds, Q, st));
             // queries with postfilter or more cells: the full graph
             if (ix->FD && opts->postfilter <= ix->P) GF_HIP(gf::launch_fullgraph(ix->rs, af, lds_f, Q, st));

@@ -54,6 +54,23 @@ inline uint32_t trav_lds_bytes(uint32_t Lpad, uint32_t hsize, uint32_t P) {
 inline uint32_t trav_dual_lds_bytes(uint32_t Lpad, uint32_t hsize) {
     return Lpad * 8 + 2 * kXSlots * 8 + 128 * 4 + hsize * 4;
 }
+// The dual channel's visited set holds rows: a bit per row (bits 0: the hash
+// table alone) for batches of up to `most` traversed queries, as many as the
+// chip holds at once with the bits in LDS, and the hash table beyond, whose
+// waves are smaller.  Whole passes, hash table against bits, u8 rows: 250k
+// rows, L = 600, 560 queries traversed 11.8 -> 9.1 ms; 250k, L = 100, 800
+// queries 1.65 -> 1.49 ms; 60k, L = 300, 3000 queries 5.07 -> 4.03 ms; over
+// the line 250k, L = 100, 4000 queries 1.85 -> 3.58 ms, 300k, L = 64, 10k
+// queries 2.48 -> 6.11 ms.
+struct VisitedRows {
+    uint32_t words, bits, most;
+};
+inline VisitedRows visited_rows(uint32_t N, uint32_t Lpad, uint32_t ncu) {
+    const uint32_t words = uint32_t((uint64_t(N) + 2047u) / 2048u * 64u);
+    if (words > 16384u) return {0u, 0u, 0u};
+    const uint32_t lds = trav_dual_lds_bytes(Lpad, words);
+    return lds <= 64u * 1024u ? VisitedRows{words, words * 32u, 160u * 1024u / lds * ncu} : VisitedRows{0u, 0u, 0u};
+}
 constexpr uint32_t kMaxAttr = 8;      // attributes per point supported
 constexpr uint32_t kAttrPad = 4;      // floats behind the attribute array: a row's attributes are read in 16-byte loads
 constexpr uint32_t kMaxE = 4;         // cross edges per (point, cell) supported
@@ -113,7 +130,8 @@ struct TravArgs {
     float* out_dist;          // Q*K
     uint32_t* counters;       // Q*GF_NCOUNTERS
     uint32_t a, P, R, E, L, K, rl, hsize, Lpad;   // hsize: visited-set words (visited_set, visited_slots)
-    uint32_t vbits;           // k_traverse: ids of the visited set's bit form (0: hash table)
+    uint32_t vbits;           // ids (k_traverse_dual: rows) of the visited set's bit form (0: hash table)
+    uint32_t qmin, qmax;      // k_traverse_dual: the launch runs when the schedule holds qmin to qmax queries
     uint32_t offl;            // 1: the launch's LDS holds the P + 1 cell offsets (trav_lds_bytes)
     // Full-graph route (queries with postfilter or more cells): the graph
     // over every point, FD rows per row (cell-major rows, kEmpty = no edge),

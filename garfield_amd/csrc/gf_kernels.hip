@@ -780,6 +780,19 @@ __device__ void hash_add_rows(uint32_t* H, uint32_t hsize, const uint64_t* A, ui
     wave_sync();
 }
 
+// The same into the dual-channel traversal's visited set, keyed by row.
+__device__ __forceinline__ void vis_add_rows(uint32_t* H, uint32_t hsize, uint32_t vbits, const uint64_t* A, uint32_t L) {
+    if (!vbits) {
+        hash_add_rows(H, hsize, A, L);
+        return;
+    }
+    for (uint32_t i = lane_id(); i < L; i += 64u) {
+        const uint64_t c = A[i];
+        if (cvalid(c)) atomicOr(&H[crow(c) >> 5], 1u << (crow(c) & 31u));
+    }
+    wave_sync();
+}
+
 // Insert the cell-local keys of A[0..L) and of one more candidate per lane
 // into the visited set, U list entries per lane at a time (a set: the order
 // of the insertions does not change membership).
@@ -1152,10 +1165,10 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
     uint32_t* S = reinterpret_cast<uint32_t*>(X + kXSlots);  // 128 row list
     uint32_t* H = S + 128;                              // visited set (rows)
     const uint32_t lane = lane_id();
-    const uint32_t si = p.srange[0] + blockIdx.x;
-    if (si >= p.srange[1]) return;
+    const uint32_t si = p.srange[0] + blockIdx.x, nq = p.srange[1] - p.srange[0];
+    if (blockIdx.x >= nq || nq < p.qmin || nq > p.qmax) return;
     const uint32_t q = p.sched[si];
-    const uint32_t hsize = p.hsize;
+    const uint32_t hsize = p.hsize, vbits = p.vbits;
     const uint32_t L = p.L, R = p.R, P = p.P, E = p.E, R2 = 2u * p.R;
 
     QReg<VT, LPR, CPL> qv;
@@ -1167,7 +1180,7 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
         hi[d] = d < p.a ? p.hi[size_t(q) * p.a + d] : 0.0f;
     }
     for (uint32_t i = lane; i < L; i += 64u) A[i] = kCandSent;
-    hash_clear(H, hsize);   // ends with a wave_sync
+    vis_clear(H, hsize, vbits);   // ends with a wave_sync
     uint32_t n_expand = 0, n_dist = 0, n_cross = 0;
     uint64_t rc = kCandSent, bleft = kCandSent;
 
@@ -1193,7 +1206,7 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
                 const bool ch1 = i >= L2;
                 const uint32_t o = ch1 ? off1 : off0, sz = (ch1 ? end1 : end0) - o;
                 row = o + p.entry[i] % sz;
-                hash_insert(H, p.hsize, row);
+                vis_insert(H, hsize, vbits, row);
                 pass = row_pass(p.attrs, p.a, row, lo, hi);
             }
             wave_sync();
@@ -1210,16 +1223,18 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
     uint32_t cur = cnt >= 2 ? 2u : 1u, turn = 0, scan0 = 0, scan1 = 0;
     for (uint32_t ep = 0; ep < kMaxIter; ++ep) {
         if ((ep + 1) % kHashReset == 0) {              // gpu_graph.cu:6364-6378
-            hash_clear(H, hsize);
-            hash_add_rows(H, p.hsize, A, L);
-            if (cvalid(bleft)) hash_insert(H, p.hsize, crow(bleft));
+            vis_clear(H, hsize, vbits);
+            vis_add_rows(H, hsize, vbits, A, L);
+            if (cvalid(bleft)) vis_insert(H, hsize, vbits, crow(bleft));
             wave_sync();
         }
         // Selection and partner (gpu_graph.cu:6380-6420).
         const uint32_t tlo = same ? 0u : (turn ? off1 : off0);
         const uint32_t thi = same ? 0xFFFFFFFFu : (turn ? end1 : end0);
         const uint32_t sel = first_unexplored_in(A, L, turn ? scan1 : scan0, tlo, thi);
-        uint32_t te_row = kEmpty, pt_row = kEmpty;
+        uint32_t te_row = kEmpty, pt_row = kEmpty, nb = 0;   // nb: the neighbour in this lane's slot
+        const uint32_t ch = lane < R ? 0u : 1u, j = lane - ch * R;
+        const bool mine = lane < R2;
         if (sel < L) {
             const uint64_t sc = A[sel];
             wave_sync();
@@ -1229,16 +1244,23 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
             else if (turn) scan1 = sel + 1;
             else scan0 = sel + 1;
             te_row = crow(sc);
-            const uint32_t oc = turn ? c0 : c1, ooff = turn ? off0 : off1;
+            const uint32_t oc = turn ? c0 : c1, ooff = turn ? off0 : off1, oend = turn ? end0 : end1;
             const uint32_t ne = E < 2u ? E : 2u;
             uint32_t v = 0;
-            bool free = false;
-            if (lane < ne) {
-                v = p.cross[size_t(te_row) * p.xrow + size_t(oc) * p.xcell + lane];
-                free = !hash_contains(H, p.hsize, p.prow[v]);
-            }
+            if (lane < ne) v = p.cross[size_t(te_row) * p.xrow + size_t(oc) * p.xcell + lane];
+            // The entry's neighbours wait for nothing, the neighbours of both
+            // possible partners only for their ids: loaded beside the test of
+            // which one it is, not after it.
+            const bool tlane = mine && ch == turn, plane = mine && ch != turn;
+            if (tlane) nb = p.graph[size_t(te_row) * R + j];
+            const uint32_t v0 = readlane32(v, 0), v1 = ne > 1u ? readlane32(v, 1) : v0;
+            uint32_t n0 = 0, n1 = 0;
+            if (plane && v0 < oend - ooff) n0 = p.graph[size_t(ooff + v0) * R + j];
+            if (plane && v1 < oend - ooff) n1 = p.graph[size_t(ooff + v1) * R + j];
+            const bool free = lane < ne && !vis_contains(H, hsize, vbits, p.prow[v]);
             const uint64_t m = ballot(free);
-            if (m) pt_row = ooff + readlane32(v, __builtin_ctzll(m));
+            if (m) pt_row = ooff + ((m & 1u) ? v0 : v1);
+            if (plane) nb = (m & 1u) ? n0 : n1;
         }
         if (sel == L) {                                 // gpu_graph.cu:6422-6547
             if (cur == cnt && same) break;
@@ -1260,7 +1282,7 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
                 const bool v = lane < L && cvalid(c) && h < E;
                 uint32_t row = 0;
                 if (v) row = offx + p.cross[size_t(crow(c)) * p.xrow + size_t(nxt) * p.xcell + h];
-                const bool isnew = v && hash_insert(H, p.hsize, row);
+                const bool isnew = v && vis_insert(H, hsize, vbits, row);
                 wave_sync();
                 n_cross += __popcll(ballot(isnew));
                 float d;
@@ -1323,16 +1345,15 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
         // of channel 1; the partner channel's last slot holds the partner.
         uint32_t row = 0;
         bool v = false;
-        if (lane < R2) {
-            const uint32_t ch = lane < R ? 0u : 1u, j = lane - ch * R;
+        if (mine) {
             const uint32_t erow = ch == turn ? te_row : pt_row;
             if (erow != kEmpty) {
                 v = true;
                 if (ch != turn && j == R - 1u) row = erow;
-                else row = (ch ? off1 : off0) + p.graph[size_t(erow) * R + j];
+                else row = (ch ? off1 : off0) + nb;
             }
         }
-        const bool isnew = v && hash_insert(H, p.hsize, row);
+        const bool isnew = v && vis_insert(H, hsize, vbits, row);
         n_expand += (te_row != kEmpty) + (pt_row != kEmpty);
         float d;
         bool pass = false;
