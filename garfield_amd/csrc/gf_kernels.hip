@@ -1232,9 +1232,7 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
         const uint32_t tlo = same ? 0u : (turn ? off1 : off0);
         const uint32_t thi = same ? 0xFFFFFFFFu : (turn ? end1 : end0);
         const uint32_t sel = first_unexplored_in(A, L, turn ? scan1 : scan0, tlo, thi);
-        uint32_t te_row = kEmpty, pt_row = kEmpty, nb = 0;   // nb: the neighbour in this lane's slot
-        const uint32_t ch = lane < R ? 0u : 1u, j = lane - ch * R;
-        const bool mine = lane < R2;
+        uint32_t te_row = kEmpty, pt_row = kEmpty;
         if (sel < L) {
             const uint64_t sc = A[sel];
             wave_sync();
@@ -1244,23 +1242,16 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
             else if (turn) scan1 = sel + 1;
             else scan0 = sel + 1;
             te_row = crow(sc);
-            const uint32_t oc = turn ? c0 : c1, ooff = turn ? off0 : off1, oend = turn ? end0 : end1;
+            const uint32_t oc = turn ? c0 : c1, ooff = turn ? off0 : off1;
             const uint32_t ne = E < 2u ? E : 2u;
             uint32_t v = 0;
-            if (lane < ne) v = p.cross[size_t(te_row) * p.xrow + size_t(oc) * p.xcell + lane];
-            // The entry's neighbours wait for nothing, the neighbours of both
-            // possible partners only for their ids: loaded beside the test of
-            // which one it is, not after it.
-            const bool tlane = mine && ch == turn, plane = mine && ch != turn;
-            if (tlane) nb = p.graph[size_t(te_row) * R + j];
-            const uint32_t v0 = readlane32(v, 0), v1 = ne > 1u ? readlane32(v, 1) : v0;
-            uint32_t n0 = 0, n1 = 0;
-            if (plane && v0 < oend - ooff) n0 = p.graph[size_t(ooff + v0) * R + j];
-            if (plane && v1 < oend - ooff) n1 = p.graph[size_t(ooff + v1) * R + j];
-            const bool free = lane < ne && !vis_contains(H, hsize, vbits, p.prow[v]);
+            bool free = false;
+            if (lane < ne) {
+                v = p.cross[size_t(te_row) * p.xrow + size_t(oc) * p.xcell + lane];
+                free = !vis_contains(H, hsize, vbits, p.prow[v]);
+            }
             const uint64_t m = ballot(free);
-            if (m) pt_row = ooff + ((m & 1u) ? v0 : v1);
-            if (plane) nb = (m & 1u) ? n0 : n1;
+            if (m) pt_row = ooff + readlane32(v, __builtin_ctzll(m));
         }
         if (sel == L) {                                 // gpu_graph.cu:6422-6547
             if (cur == cnt && same) break;
@@ -1345,12 +1336,13 @@ __global__ __launch_bounds__(64) void k_traverse_dual(TravArgs p) {
         // of channel 1; the partner channel's last slot holds the partner.
         uint32_t row = 0;
         bool v = false;
-        if (mine) {
+        if (lane < R2) {
+            const uint32_t ch = lane < R ? 0u : 1u, j = lane - ch * R;
             const uint32_t erow = ch == turn ? te_row : pt_row;
             if (erow != kEmpty) {
                 v = true;
                 if (ch != turn && j == R - 1u) row = erow;
-                else row = (ch ? off1 : off0) + nb;
+                else row = (ch ? off1 : off0) + p.graph[size_t(erow) * R + j];
             }
         }
         const bool isnew = v && vis_insert(H, hsize, vbits, row);
