@@ -407,19 +407,23 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
         bool ints = ix.sub && !gf::half_rows(ix.vdtype) && ix.vdtype != GF_VEC_I8Q && D <= 256;
         for (size_t i = 0; ints && i < v.size(); ++i) ints = v[i] >= 0.0f && v[i] <= 255.0f && v[i] == std::floor(v[i]);
         if (ints) {
-            ix.Db = gf::bf_i8_dim(D);
-            ix.trec.alloc(size_t(ix.ntile) * gf::bf_rec_bytes(ix.Db, ix.AW));
+            ix.Db8 = gf::bf_i8_dim(D);
+            ix.trec.alloc(size_t(ix.ntile) * gf::bf_rec_bytes(ix.Db8, ix.AW));
             GF_HIP(gf::launch_tile_rec(vec_f32_dev, false, D, ix.tmeta.p, ix.AW, ix.ntile, ix.trec.p,
                                       ix.stream));
             ix.i8 = true;
         }
-        // Float rows with sub-cells and no int8 route: |x|^2 per row (fp32:
-        // binary16 rows as k_norms_f16 sums their values, fp32 rows from a
-        // float64 sum) and the largest |x| for the MFMA brute force's error
-        // bound (a binary16 value is within 2^-11 of x * alpha, or 2^-25 for
-        // subnormals).
+        // Float rows with sub-cells: |x|^2 per row (fp32: binary16 rows as
+        // k_norms_f16 sums their values, fp32 rows from a float64 sum) and
+        // the largest |x| for the MFMA brute force's error bound (a binary16
+        // value is within 2^-11 of x * alpha, or 2^-25 for subnormals).
+        // Integer-valued rows take the int8 route alone, except at the
+        // dimension that only that route pads (96): there batches of
+        // non-integer queries run here (250k points, 4000 queries: 0.75 ms
+        // a search against 8.7 ms of the gather kernel).
         const int fvt = ix.vdtype == GF_VEC_F16 ? 1 : (ix.vdtype == GF_VEC_F32 ? 0 : -1);
-        if (ix.sub && !ix.i8 && fvt >= 0 && gf::bf_float_supported(fvt, D, ix.AW, 1)) {
+        const bool floats = !ix.i8 || (ix.Db8 != D && gf::bf_float_dim(fvt, D) == D);
+        if (ix.sub && floats && fvt >= 0 && gf::bf_float_supported(fvt, D, ix.AW, 1)) {
             std::vector<float> xn(fvt == 0 ? N : 0);
             double xm = 0.0;
             for (uint32_t r = 0; r < N; ++r) {
@@ -442,10 +446,10 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
             }
             // the brute force's tile records: its tiles' rows in MFMA operand
             // order, contiguous per tile, with their meta records and norms
-            ix.Db = gf::bf_float_dim(fvt, D);
-            const uint32_t KS = fvt == 1 ? ix.Db / 32 : ix.Db / 16;
+            ix.Dbf = gf::bf_float_dim(fvt, D);
+            const uint32_t KS = fvt == 1 ? ix.Dbf / 32 : ix.Dbf / 16;
             ix.frec.alloc(size_t(ix.ntile) * gf::bf_frec_bytes(KS, ix.AW));
-            GF_HIP(gf::launch_tile_frec(ix.vec.p, fvt, D, ix.Db, ix.tmeta.p, ix.xnormf.p, ix.AW, ix.ntile, ix.frec.p,
+            GF_HIP(gf::launch_tile_frec(ix.vec.p, fvt, D, ix.Dbf, ix.tmeta.p, ix.xnormf.p, ix.AW, ix.ntile, ix.frec.p,
                                         ix.stream));
             ix.hf = true;
             // Binary16 rows' first pass (a launch of its own): one in four
@@ -821,7 +825,19 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             b->q16v.alloc(size_t(Q) * ix->D);
             GF_HIP(gf::launch_f2h(b->qf32.p, b->q16v.p, size_t(Q) * ix->D, ix->alpha, ix->stream));
         }
-        if (ix->hf) {
+        if (ix->i8) {
+            bool ints = true;
+            const size_t nq = size_t(Q) * ix->D;
+            for (size_t i = 0; ints && i < nq; ++i)
+                ints = queries[i] >= 0.0f && queries[i] <= 255.0f && queries[i] == std::floor(queries[i]);
+            if (ints) {
+                b->q8.alloc(size_t(Q) * ix->Db8);
+                b->nq.alloc(Q);
+                GF_HIP(gf::launch_q_i8(b->qf32.p, Q, ix->D, ix->Db8, b->q8.p, b->nq.p, ix->stream));
+                b->i8 = true;
+            }
+        }
+        if (ix->hf && !b->i8) {
             // |q|^2 of the query as the rows hold it (binary16 or fp32), and
             // the bound eps_q of |d' - d| for the MFMA brute force of float
             // rows: d' = |q|^2 + |x|^2 - 2 q.x and the canonical d each hold
@@ -831,7 +847,7 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             // products.
             const uint32_t D = ix->D;
             const bool h = ix->vdtype == GF_VEC_F16;
-            const double u = std::ldexp(1.0, -24), gam = (ix->Db + 2) * u / (1.0 - (ix->Db + 2) * u);
+            const double u = std::ldexp(1.0, -24), gam = (ix->Dbf + 2) * u / (1.0 - (ix->Dbf + 2) * u);
             std::vector<float> eps(Q), qn(h ? 0 : Q);
             for (uint32_t q = 0; q < Q; ++q) {
                 double s = 0.0;
@@ -853,12 +869,12 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
                 b->qnf.upload(qn);
             }
             b->heps.upload(eps);
-            if (ix->Db != D) {
+            if (ix->Dbf != D) {
                 // the kernel's queries, zero padded to the records' dimension
                 const size_t es = h ? 2 : 4;
-                b->qpad.alloc(size_t(Q) * ix->Db * es);
+                b->qpad.alloc(size_t(Q) * ix->Dbf * es);
                 GF_HIP(hipMemsetAsync(b->qpad.p, 0, b->qpad.n, ix->stream));
-                GF_HIP(hipMemcpy2DAsync(b->qpad.p, ix->Db * es,
+                GF_HIP(hipMemcpy2DAsync(b->qpad.p, ix->Dbf * es,
                                         h ? static_cast<const void*>(b->q16v.p) : static_cast<const void*>(b->qf32.p),
                                         D * es, D * es, Q, hipMemcpyDeviceToDevice, ix->stream));
             }
@@ -881,18 +897,6 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             GF_HIP(gf::launch_f2h_pad(b->qf32.p, Q, ix->D, b->q16.p, b->Qp, ix->Dp, ix->alpha, ix->stream));
             b->qnorm.alloc(b->Qp);
             GF_HIP(gf::launch_norms_f16(b->q16.p, b->Qp, ix->Dp, ix->Dp, b->qnorm.p, ix->stream));
-        }
-        if (ix->i8) {
-            bool ints = true;
-            const size_t nq = size_t(Q) * ix->D;
-            for (size_t i = 0; ints && i < nq; ++i)
-                ints = queries[i] >= 0.0f && queries[i] <= 255.0f && queries[i] == std::floor(queries[i]);
-            if (ints) {
-                b->q8.alloc(size_t(Q) * ix->Db);
-                b->nq.alloc(Q);
-                GF_HIP(gf::launch_q_i8(b->qf32.p, Q, ix->D, ix->Db, b->q8.p, b->nq.p, ix->stream));
-                b->i8 = true;
-            }
         }
         b->cells.alloc(size_t(Q) * ix->P);
         b->counts.alloc(Q);
@@ -1154,7 +1158,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     // Brute-force route on MFMA when vectors and queries are int8-exact:
     // work items of (sub-cell, <= 64 queries whose range reaches it),
     // scheduled on the device.
-    // Dimensions that run padded (Db > D) take it for larger batches only:
+    // Dimensions that run padded (Db8, Dbf > D) take it for larger batches only:
     // below these lines the gather kernel's parts finish before the MFMA
     // route's chain of launches would.  rows x (row bytes + 160) is the
     // gather's cost if every row passes; measured at 100 dimensions, all rows
@@ -1163,13 +1167,16 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     // 220; fp32 6M rows (3.4 GB) 398 / 179 against 384 / 326, 12M rows 711 /
     // 242 against 417 / 342.
     const double gather_bytes = double(Q) * ix->N * (ix->rowbytes + 160.0);
-    const bool padded = ix->Db != ix->D;
-    const bool gemm = ix->i8 && b->i8 && K <= gf::kBfKMax && !(padded && gather_bytes < 1.8e9);
+    const bool gemm = ix->i8 && b->i8 && K <= gf::kBfKMax && !(ix->Db8 != ix->D && gather_bytes < 1.8e9);
     // Binary16 rows: the same items on fp16 MFMA, candidates within the
     // distances' error bound re-ranked exactly (k_bf_f16, k_bf_f16_final).
     const int fvt = ix->vdtype == GF_VEC_F16 ? 1 : 0;
+    // Non-integer queries over integer-valued rows (96 dimensions) take it
+    // from the size where it is no slower than the gather kernel at 1 to 50 %
+    // passing: 100k points, 100 queries (5.4 GB) 320 us against 193, 250k,
+    // 300 (41 GB) 330 against 1000, 250k, 4000 0.73 ms against 8.7 ms.
     const bool gemm_h = !gemm && ix->hf && b->qnf.n == Q && gf::bf_float_supported(fvt, ix->D, ix->AW, K) &&
-                        !(padded && gather_bytes < 3.4e9);
+                        !(ix->Dbf != ix->D && gather_bytes < 3.4e9) && !(ix->i8 && gather_bytes < 7e9);
     const bool sched_bf = gemm || gemm_h;
     const uint32_t KP = gemm_h ? gf::kBfHKT : K;   // keys per (query, item) in the partial area
     const uint32_t seed_tiles = gemm_h ? gf::kBfHSeedTiles : gf::kBfSeedTiles;
@@ -1285,7 +1292,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             ha.pcnt = b->pcnt.p; ha.part = b->part.p; ha.gbound = b->gbound.p; ha.over = b->hover.p;
             ha.ok = tot + 3;
             if (seeds) { ha.sitems = b->sitems.p; ha.nseed = tot + 5; ha.nseed_cap = scap; ha.seeds_on = 1; }
-            ha.K = K; ha.D = ix->Db;
+            ha.K = K; ha.D = ix->Dbf;
             GF_HIP(gf::launch_stamp(stamp + 3, st));
             // Binary16 rows: the seeds alone, then (two passes) the
             // first-pass sub-cells' items, then the rest, each launch
@@ -1323,7 +1330,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         ga.part_off = b->part_off.p; ga.part = b->part.p; ga.gbound = b->gbound.p;
         ga.ok = tot + 3;
         if (seeds) { ga.sitems = b->sitems.p; ga.nseed = tot + 5; ga.nseed_cap = scap; ga.seeds_on = 1; }
-        ga.K = K; ga.D = ix->Db;
+        ga.K = K; ga.D = ix->Db8;
         gf::BfFinalArgs fa{};
         fa.gbound = b->gbound.p; fa.bfq = b->sched.p; fa.srange = tot + 14; fa.part_off = b->part_off.p; fa.pcnt = b->pcnt.p;
         fa.ok = tot + 3; fa.part = b->part.p; fa.counts = b->counts.p; fa.cells = b->cells.p;
@@ -1547,7 +1554,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // Item schedule: every (query, sub-cell) pair costs 2 D ops per
             // point; every item streams its sub-cell's tiles once; the final
             // merge reads the appended keys.
-            const double tile_bytes = (ix->Db / 64) * 1024.0 + 32 * 4.0 + 16.0 * (1 + ix->AW) * 4.0;
+            const double tile_bytes = (ix->Db8 / 64) * 1024.0 + 32 * 4.0 + 16.0 * (1 + ix->AW) * 4.0;
             stats->ops_bruteforce = 2.0 * ix->D * double(sm[9]);
             stats->bytes_bruteforce = double(sm[10]) * tile_bytes + double(dt[9]) * K * 16.0;
             stats->bf_mfma = 1;
@@ -1555,7 +1562,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // fp16 items: every (query, sub-cell) pair costs 2 D flops per
             // point; every item streams its sub-cell's rows and meta; the
             // final re-rank gathers the candidates' rows
-            const double tile_bytes = 16.0 * ix->Db * 2.0 + 16.0 * (2 + ix->AW) * 4.0;
+            const double tile_bytes = 16.0 * ix->Dbf * 2.0 + 16.0 * (2 + ix->AW) * 4.0;
             stats->ops_bruteforce = 2.0 * ix->D * double(sm[9]);
             stats->bytes_bruteforce = double(sm[10]) * tile_bytes + b_dist * ix->rowbytes + double(dt[9]) * K * 16.0;
             stats->bf_mfma = 2;

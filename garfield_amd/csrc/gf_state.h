@@ -240,7 +240,7 @@ struct gf_index {
     gf::RowShape rs{};
     uint32_t rowbytes = 0, Cp = 0, Dp = 0;
     uint32_t max_cell = 0;   // points of the largest cell
-    uint32_t Db = 0;         // dimension of the MFMA brute force's records (bf_i8_dim, bf_float_dim)
+    uint32_t Db8 = 0, Dbf = 0;   // dimensions of the MFMA brute force's int8 and float records (bf_i8_dim, bf_float_dim)
     std::vector<uint32_t> offset_h, grid_h;
     DevBuf<char> vec;
     DevBuf<float> attrs, l_q, r_q, cnorm;
@@ -272,8 +272,9 @@ struct gf_index {
     bool i8 = false;
     DevBuf<uint8_t> trec;   // MFMA brute force: int8 tile records (gf::bf_rec_bytes each)
     // Float rows with sub-cells (binary16 or fp32, shapes of
-    // bf_float_supported) and no int8 route: the MFMA brute force of float
-    // rows, with |x|^2 per row and the largest |x| over the index.
+    // bf_float_supported): the MFMA brute force of float rows, with |x|^2 per
+    // row and the largest |x| over the index.  Integer-valued rows have it
+    // beside the int8 route where only that one pads (96 dimensions).
     bool hf = false;
     DevBuf<float> xnormf;
     DevBuf<uint8_t> frec;   // its tile records (gf::bf_frec_bytes each)
@@ -421,7 +422,7 @@ struct gf_batch {
     DevBuf<uint16_t> q16, q16v;
     DevBuf<float> qi8q;   // GF_VEC_I8Q: query rows [c | s], c_d = fma(s_d, z_d, q_d)
     DevBuf<float> qnf, heps;   // float MFMA brute force: |q|^2 of the query as the rows hold it, bound of |d' - d|
-    DevBuf<char> qpad;          // float MFMA brute force: queries zero padded to Db dimensions
+    DevBuf<char> qpad;          // float MFMA brute force: queries zero padded to Dbf dimensions
     DevBuf<uint64_t> bfs_keys;  // gather brute force in parts (gf::BfSplit)
     DevBuf<uint32_t> bfs_cnt;
     DevBuf<uint32_t> hover;     // fp16 brute force: queries whose kept keys may miss a candidate

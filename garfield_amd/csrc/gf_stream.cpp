@@ -434,7 +434,7 @@ void build_streamed(const gf_index_host& h, const gf_open_opts* opts, const gf_s
         std::vector<uint32_t>().swap(S.sh.sorder);
         std::vector<uint32_t>().swap(S.sh.scell);
         ix.i8 = true;   // gf_batch_create keeps int8 queries
-        ix.Db = bf_i8_dim(D);
+        ix.Db8 = bf_i8_dim(D);
     }
     GF_HIP(hipDeviceGetAttribute(&ix.ncu, hipDeviceAttributeMultiprocessorCount, ix.device));
     ix.offset.upload(ix.offset_h);
