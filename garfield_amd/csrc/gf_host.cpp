@@ -74,6 +74,7 @@ void build_subcells(const gf_index_host& h, const std::vector<uint32_t>& gidx, c
     ix.ntile = sh.ntile;
     ix.ssize_h = sh.ssize;
     ix.stile_h = sh.stile;
+    for (uint32_t s = 0; s < ix.NS; ++s) ix.tmax = std::max(ix.tmax, ix.stile_h[s + 1] - ix.stile_h[s]);
     ix.abase.upload(sh.abase);
     ix.sbase.upload(sh.sbase);
     ix.scell.upload(sh.scell);
@@ -84,6 +85,9 @@ void build_subcells(const gf_index_host& h, const std::vector<uint32_t>& gidx, c
     ix.sorder.upload(sh.sorder);
     ix.ns1 = sh.ns1;
     ix.shash_h = std::move(sh.shash);
+    ix.sbox_h.resize(sh.sbox.size());
+    for (uint32_t s = 0; s < ix.NS; ++s)
+        for (uint32_t j = 0; j < 2 * ix.a; ++j) ix.sbox_h[size_t(j) * ix.NS + s] = float(sh.sbox[size_t(s) * 2 * ix.a + j]);
     ix.sub = true;
 }
 
@@ -807,6 +811,34 @@ gf_status gf_index_get_info(const gf_index* ix, gf_index_info* out) {
     });
 }
 
+// The first size of the batch's pair lists, from what the ranges of up to
+// kBfReach of its queries reach: those that stage A can send to the brute force
+// (their sub-cells, which hold their points and some beside them, no more than
+// twice its share of the tiles).
+static size_t first_pairs(const gf_batch& b, uint32_t tch, uint32_t seed_tiles, uint32_t kp) {
+    const gf_index& ix = *b.ix;
+    const uint32_t a = ix.a, NS = ix.NS, n = uint32_t(b.reach_lo.size() / a);
+    std::vector<uint32_t> hit(NS);
+    uint64_t chunks = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        std::fill(hit.begin(), hit.end(), 1u);
+        for (uint32_t d = 0; d < a; ++d) {
+            const float lo = b.reach_lo[size_t(i) * a + d], hi = b.reach_hi[size_t(i) * a + d];
+            const float *mn = &ix.sbox_h[size_t(2 * d) * NS], *mx = mn + NS;
+            for (uint32_t s = 0; s < NS; ++s) hit[s] &= uint32_t(hi >= mn[s]) & uint32_t(mx[s] >= lo);
+        }
+        uint64_t tiles = 0, c = 0;
+        for (uint32_t s = 0; s < NS; ++s) {
+            if (!hit[s]) continue;
+            const uint32_t t = ix.stile_h[s + 1] - ix.stile_h[s];
+            tiles += t;
+            c += (t + tch - 1) / tch;
+        }
+        if (b.prefilter >= 1.0f || double(tiles) <= 2.0 * b.prefilter * ix.ntile) chunks += c;
+    }
+    return gf::bf_first_pairs(b.Q, chunks, n, ix.tmax, seed_tiles, kp);
+}
+
 gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const float* lo, const float* hi,
                           gf_batch** out) {
     return run_guarded([&] {
@@ -898,6 +930,14 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             b->qnorm.alloc(b->Qp);
             GF_HIP(gf::launch_norms_f16(b->q16.p, b->Qp, ix->Dp, ix->Dp, b->qnorm.p, ix->stream));
         }
+        if (!ix->sx && (b->i8 || b->qnf.n)) {
+            const uint32_t n = std::min(Q, gf::kBfReach);
+            for (uint32_t i = 0; i < n; ++i) {
+                const size_t at = size_t(uint64_t(i) * Q / n) * ix->a;
+                b->reach_lo.insert(b->reach_lo.end(), lo + at, lo + at + ix->a);
+                b->reach_hi.insert(b->reach_hi.end(), hi + at, hi + at + ix->a);
+            }
+        }
         b->cells.alloc(size_t(Q) * ix->P);
         b->counts.alloc(Q);
         b->little.alloc(Q);
@@ -938,6 +978,7 @@ gf_status gf_mark_cells(gf_batch* b, float prefilter, double* ms) {
         b->bf_all = true;
         b->sel_exact = count;
         b->route_bf = !count;
+        b->prefilter = prefilter;
         b->time_a = gf_batch::kTimeStamps;
         b->marked = true;
         if (!ms) {
@@ -982,6 +1023,7 @@ gf_status gf_mark_cells_grid(gf_batch* b, const float* attr_min, const float* at
         b->flags_ready = true;
         b->bf_all = false;
         b->route_bf = false;
+        b->prefilter = 1.0f;
         b->sel_exact = true;   // the arithmetic-grid stage A counts nothing: selcount stays 0
     });
 }
@@ -1191,7 +1233,8 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
         // item slots: a sub-cell adds up to two partial query blocks per
         // tile chunk beyond pairs / 64
         const size_t islots = size_t(NS) + ix->ntile / tch + 1;
-        if (!b->part.n) b->alloc_pairs(size_t(Q) * 64, KP, Q, NS, islots);
+        if (!b->part.n)
+            b->alloc_pairs(first_pairs(*b, tch, seed_tiles, KP), KP, Q, NS, islots);
         if (b->rq.n < Q) {
             b->rq.alloc(Q); b->rseed.alloc(Q);
             b->rlo.alloc(size_t(Q) * ix->a); b->rhi.alloc(size_t(Q) * ix->a);
@@ -1201,10 +1244,8 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
             // a seed sub-cell s with ns queries makes ceil(ns / 64) items per
             // chunk of seed tiles (sized for the smaller chunk of the two
             // routes); every query seeds one sub-cell
-            uint32_t tmax = 0;
-            for (uint32_t s = 0; s < NS; ++s) tmax = std::max(tmax, ix->stile_h[s + 1] - ix->stile_h[s]);
             const uint32_t sch = std::min(gf::kBfSeedTiles, gf::kBfHSeedTiles);
-            const size_t chunks = (tmax + sch - 1) / sch;
+            const size_t chunks = (ix->tmax + sch - 1) / sch;
             b->sitems.alloc((size_t(Q) / gf::kBfQB + NS + 1) * std::max<size_t>(chunks, 1));
         }
         if (b->part.n < b->pair_cap * KP) b->part.alloc(b->pair_cap * KP);
@@ -1633,6 +1674,7 @@ gf_status gf_batch_set_cells(gf_batch* b, const uint32_t* cells, const uint32_t*
         b->flags_ready = false;
         b->bf_all = false;
         b->route_bf = false;
+        b->prefilter = 1.0f;
     });
 }
 

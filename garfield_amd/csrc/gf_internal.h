@@ -185,6 +185,26 @@ inline uint32_t bf_item_tiles(uint32_t NS, uint32_t Q) {
 // 1M points, 10k queries 7.32 -> 5.68 ms; 768-d binary16, 120k points, 4096
 // queries 914 -> 733 us, 400k points, 10k queries 2.38 -> 2.42 ms.
 constexpr uint32_t kBfHItemTiles = 48;
+// Pairs that a batch's lists are first made for, a pair being a (query,
+// sub-cell) combination of one chunk of at most tch tiles: the chunks that n of
+// the batch's Q queries reach, over n, and a seed's, and a fifth more; 64 a
+// query at least and kBfPairBytes of partial results (kp keys a pair) at most.
+// Lists that do not fit cost their search a wait, new buffers and a second
+// brute force.  A buffer of more than kFastFreeBytes takes 250 us to free, a
+// smaller one 12, so the fifth ends there.  New batches, 128-d integers, at 64
+// pairs a query against this: 100k points, 500 queries 1470 -> 730 us, 2000
+// queries 1760 -> 1010 us, 250k points, 4000 queries 1890 -> 1740 us (1380
+// with whole sub-cells, whose pairs take 20 MB and not 70), 400k points, 4000
+// queries 2160 -> 1490 us.
+constexpr size_t kBfPairBytes = size_t(1) << 30, kFastFreeBytes = size_t(64) << 20;
+constexpr uint32_t kBfReach = 64;   // queries whose reach is looked at
+inline size_t bf_first_pairs(uint32_t Q, uint64_t chunks, uint32_t n, uint32_t tmax, uint32_t seed_tiles, uint32_t kp) {
+    const size_t key = size_t(kp) * sizeof(uint64_t), most = kBfPairBytes / key, fast = kFastFreeBytes / key;
+    const size_t least = size_t(Q) * 64, seed = (size_t(tmax) + seed_tiles - 1u) / seed_tiles;
+    const size_t seen = (n ? size_t(Q) * chunks / n : 0) + Q * seed;
+    const size_t want = seen <= fast && seen + seen / 5 > fast ? fast : seen + seen / 5;
+    return want < least ? least : want <= most ? want : least > most ? least : most;
+}
 constexpr uint32_t kBfSeedTiles = 16;         // tiles per seed item: a seed sub-cell spreads over several waves
 constexpr uint32_t kBfHFirstPass = 4;         // binary16 rows' first pass: sub-cells with grid hash % 4 == 0
 constexpr uint32_t kBfHSeedTiles = 128;       // the same for the float MFMA route (measured: C4 5.6 ms at 128, 6.0 at 16)

@@ -261,8 +261,9 @@ struct gf_index {
     // attribute; tiles of 16 points are grouped by sub-cell and carry the
     // cell-major row and the packed 16-bit attribute offsets of each point.
     bool sub = false;
-    uint32_t AW = 0, NS = 0, ntile = 0;
+    uint32_t AW = 0, NS = 0, ntile = 0, tmax = 0;   // tmax: tiles of the longest sub-cell
     std::vector<uint32_t> ssize_h, stile_h, shash_h;
+    std::vector<float> sbox_h;   // sub-cells' smallest and largest values, NS each, per attribute
     DevBuf<uint32_t> sbase, scell, ssize, stile, tmeta;
     DevBuf<uint32_t> sorder;   // sub-cells of the brute force's first pass (ns1 of them), then the rest
     uint32_t ns1 = 0;
@@ -372,6 +373,12 @@ struct gf_batch {
     bool marked = false;
     // the latest stage A sent every query to the brute force (prefilter >= 1)
     bool route_bf = false;
+    // its prefilter (1 where it was not gf_mark_cells): the share of the
+    // points that a brute-force query's range holds, at most
+    float prefilter = 1.0f;
+    // MFMA brute force: lower and upper bounds of up to kBfReach of the
+    // queries, which size the pair lists (first_pairs)
+    std::vector<float> reach_lo, reach_hi;
     // Stage calls made without ms on a resident index, not yet enqueued:
     // the search enqueues them in its own graph; any other call that reads
     // or writes the stage buffers enqueues them first (flush_stages).
