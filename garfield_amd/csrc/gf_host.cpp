@@ -1223,7 +1223,9 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     const uint32_t KP = gemm_h ? gf::kBfHKT : K;   // keys per (query, item) in the partial area
     const uint32_t seed_tiles = gemm_h ? gf::kBfHSeedTiles : gf::kBfSeedTiles;
     const uint32_t NS = ix->NS;
-    const uint32_t tch = gemm_h ? gf::kBfHItemTiles : gf::bf_item_tiles(NS, Q);   // tiles per item, at most
+    // tiles per item, at most
+    const uint32_t tch =
+        gemm_h ? gf::bf_float_item_tiles(NS, ix->ntile, ix->tmax, Q) : gf::bf_item_tiles(NS, Q);
     b->pass_pending = sched_bf && !b->sel_exact;
     if (sched_bf) {
         if (!b->bcnt.n) {

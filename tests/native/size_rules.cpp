@@ -11,6 +11,8 @@ int main(int argc, char** argv) {
     const char* rule = argc > 1 ? argv[1] : "";
     if (!std::strcmp(rule, "first_pairs"))
         std::printf("%zu\n", gf::bf_first_pairs(u(2), u(3), u(4), u(5), u(6), u(7)));
+    else if (!std::strcmp(rule, "float_item_tiles"))
+        std::printf("%u\n", gf::bf_float_item_tiles(u(2), u(3), u(4), u(5)));
     else
         return 2;
     return 0;

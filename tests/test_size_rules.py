@@ -52,3 +52,14 @@ def test_first_pairs_are_bounded(rule):
     assert rule("first_pairs", 4000, 64 * 220, 64, 72, 16, 10) == 4000 * 225 * 6 // 5
     assert rule("first_pairs", 50_000, 64 * 400, 64, 96, 128, 32) * 32 * 8 == 1 << 30
     assert rule("first_pairs", 200_000, 64 * 400, 64, 96, 128, 32) == 200_000 * 64
+
+
+def test_float_items_are_whole_where_many_and_even(rule):
+    """Whole sub-cells from 14001 items up if none is more than twice the
+    mean, chunks of 48 tiles otherwise."""
+    whole, chunk = 65536, 48
+    assert rule("float_item_tiles", 140, 140 * 64, 96, 6400) == chunk
+    assert rule("float_item_tiles", 140, 140 * 64, 96, 6401) == whole
+    assert rule("float_item_tiles", 976, 976 * 64, 128, 10_000) == whole
+    assert rule("float_item_tiles", 976, 976 * 64, 129, 10_000) == chunk
+    assert rule("float_item_tiles", 976, 976 * 64, 96, 64) == chunk
