@@ -1200,15 +1200,24 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     // Brute-force route on MFMA when vectors and queries are int8-exact:
     // work items of (sub-cell, <= 64 queries whose range reaches it),
     // scheduled on the device.
-    // Dimensions that run padded (Db8, Dbf > D) take it for larger batches only:
-    // below these lines the gather kernel's parts finish before the MFMA
+    // Dimensions that run padded (Db8, Dbf > D) take it for larger batches
+    // only: below these lines the gather kernel's parts finish before the MFMA
     // route's chain of launches would.  rows x (row bytes + 160) is the
-    // gather's cost if every row passes; measured at 100 dimensions, all rows
-    // passing / 1 to 50 % passing, gather against MFMA: int8 3.2M rows (1.8
-    // GB) 199 / 130 us against 264 / 268, 6M rows 399 / 181 against 234 /
-    // 220; fp32 6M rows (3.4 GB) 398 / 179 against 384 / 326, 12M rows 711 /
-    // 242 against 417 / 342.
-    const double gather_bytes = double(Q) * ix->N * (ix->rowbytes + 160.0);
+    // gather's cost if every row passes.  A prefilter below 1 bounds what does:
+    // stage A sends to the brute force the queries that at most that share of
+    // the points pass, and fewer of them, so 0.6 of it is taken.  Without that
+    // bound the lines are where the two break even if every row passes; if
+    // 1 to 50 % do, the gather is up to twice as fast from there to three times
+    // the line, and the MFMA route as much faster beyond it if all do.
+    // Measured, kept batches, 1 to 50 % passing (all), gather / MFMA: int8, 100
+    // dimensions 1.4 GB 111 / 190 us (164 / 177), 4.2 GB 170 / 187 (376 / 180),
+    // 16.8 GB 438 / 216; fp32, 100 dimensions 4.2 GB 170 / 277 (379 / 371),
+    // 16.8 GB 448 / 316 (760 / 458); prefilter 0.3, int8 5.6 GB 341 / 376, 16.8
+    // GB 515 / 389, fp32 16.8 GB 504 / 495, 67 GB 1257 / 570; prefilter 0.05,
+    // int8 67 GB 403 / 412, 252 GB 826 / 543, fp32 84 GB 470 / 612, 252 GB 821 /
+    // 653 (208 dimensions of u8, 16, 200 and 264 alike).
+    const double share = b->prefilter < 1.0f ? 0.6 * b->prefilter : 1.0;
+    const double gather_bytes = share * double(Q) * ix->N * (ix->rowbytes + 160.0);
     const bool gemm = ix->i8 && b->i8 && K <= gf::kBfKMax && !(ix->Db8 != ix->D && gather_bytes < 1.8e9);
     // Binary16 rows: the same items on fp16 MFMA, candidates within the
     // distances' error bound re-ranked exactly (k_bf_f16, k_bf_f16_final).
