@@ -353,6 +353,38 @@ void entry_points_pair(uint32_t range1, uint32_t R, uint32_t range2, uint32_t BD
 
 namespace {
 
+// Whether every value is an integer in [0, 255].
+bool small_ints(const float* v, size_t n) {
+    constexpr size_t B = 4096;   // a block is tested whole: it vectorises (std::floor is a call per value)
+    for (size_t i = 0; i < n; i += B) {
+        const size_t e = std::min(n, i + B);
+        uint32_t bad = 0;
+        for (size_t j = i; j < e; ++j) {
+            const float x = v[j], y = x >= 0.0f && x <= 255.0f ? x : 0.5f;
+            bad |= uint32_t(float(int32_t(y)) != y);
+        }
+        if (bad) return false;
+    }
+    return true;
+}
+
+// |x alpha|^2 in 64 bits, in eight sums so that no addition waits for the last.
+double square_sum(const float* x, uint32_t D, float alpha) {
+    constexpr uint32_t U = 8;
+    double s[U] = {};
+    uint32_t d = 0;
+    for (; d + U <= D; d += U)
+        for (uint32_t u = 0; u < U; ++u) {
+            const double y = double(x[d + u]) * alpha;
+            s[u] += y * y;
+        }
+    for (; d < D; ++d) {
+        const double y = double(x[d]) * alpha;
+        s[0] += y * y;
+    }
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix) {
     std::vector<uint32_t> size, gidx, lrow;
     gf::map_cells(h, opts, ix, size, gidx, lrow);
@@ -407,9 +439,16 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
             vec_f32_dev = tmp.p;
         }
         build_subcells(h, gidx, size, ix);
+        auto records_fit = [&](uint32_t Dp, size_t bytes) {
+            size_t avail = 0, total = 0;
+            if (Dp == D) return true;
+            GF_HIP(hipMemGetInfo(&avail, &total));
+            return gf::bf_pad_records_fit(bytes, avail);
+        };
         // Integer-valued data in [0, 255]: int8 tiles of the MFMA brute force.
-        bool ints = ix.sub && !gf::half_rows(ix.vdtype) && ix.vdtype != GF_VEC_I8Q && D <= 256;
-        for (size_t i = 0; ints && i < v.size(); ++i) ints = v[i] >= 0.0f && v[i] <= 255.0f && v[i] == std::floor(v[i]);
+        const bool ints = ix.sub && !gf::half_rows(ix.vdtype) && ix.vdtype != GF_VEC_I8Q && D <= 256 &&
+                          small_ints(v.data(), v.size()) &&
+                          records_fit(gf::bf_i8_dim(D), size_t(ix.ntile) * gf::bf_rec_bytes(gf::bf_i8_dim(D), ix.AW));
         if (ints) {
             ix.Db8 = gf::bf_i8_dim(D);
             ix.trec.alloc(size_t(ix.ntile) * gf::bf_rec_bytes(ix.Db8, ix.AW));
@@ -427,15 +466,14 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
         // a search against 8.7 ms of the gather kernel).
         const int fvt = ix.vdtype == GF_VEC_F16 ? 1 : (ix.vdtype == GF_VEC_F32 ? 0 : -1);
         const bool floats = !ix.i8 || (ix.Db8 != D && gf::bf_float_dim(fvt, D) == D);
-        if (ix.sub && floats && fvt >= 0 && gf::bf_float_supported(fvt, D, ix.AW, 1)) {
+        const bool route = ix.sub && floats && fvt >= 0 && gf::bf_float_supported(fvt, D, ix.AW, 1);
+        const uint32_t Dbf = route ? gf::bf_float_dim(fvt, D) : 0u;
+        const uint32_t KS = fvt == 1 ? Dbf / 32 : Dbf / 16;
+        if (Dbf && records_fit(Dbf, size_t(ix.ntile) * gf::bf_frec_bytes(KS, ix.AW))) {
             std::vector<float> xn(fvt == 0 ? N : 0);
             double xm = 0.0;
             for (uint32_t r = 0; r < N; ++r) {
-                double s = 0.0;
-                for (uint32_t d = 0; d < D; ++d) {
-                    const double x = double(v[size_t(r) * D + d]) * (fvt == 1 ? ix.alpha : 1.0f);
-                    s += x * x;
-                }
+                const double s = square_sum(&v[size_t(r) * D], D, fvt == 1 ? ix.alpha : 1.0f);
                 xm = std::max(xm, s);
                 if (fvt == 0) xn[r] = float(s);
             }
@@ -450,8 +488,7 @@ void build_index(const gf_index_host& h, const gf_open_opts* opts, gf_index& ix)
             }
             // the brute force's tile records: its tiles' rows in MFMA operand
             // order, contiguous per tile, with their meta records and norms
-            ix.Dbf = gf::bf_float_dim(fvt, D);
-            const uint32_t KS = fvt == 1 ? ix.Dbf / 32 : ix.Dbf / 16;
+            ix.Dbf = Dbf;
             ix.frec.alloc(size_t(ix.ntile) * gf::bf_frec_bytes(KS, ix.AW));
             GF_HIP(gf::launch_tile_frec(ix.vec.p, fvt, D, ix.Dbf, ix.tmeta.p, ix.xnormf.p, ix.AW, ix.ntile, ix.frec.p,
                                         ix.stream));
@@ -858,11 +895,7 @@ gf_status gf_batch_create(gf_index* ix, const float* queries, uint32_t Q, const 
             GF_HIP(gf::launch_f2h(b->qf32.p, b->q16v.p, size_t(Q) * ix->D, ix->alpha, ix->stream));
         }
         if (ix->i8) {
-            bool ints = true;
-            const size_t nq = size_t(Q) * ix->D;
-            for (size_t i = 0; ints && i < nq; ++i)
-                ints = queries[i] >= 0.0f && queries[i] <= 255.0f && queries[i] == std::floor(queries[i]);
-            if (ints) {
+            if (small_ints(queries, size_t(Q) * ix->D)) {
                 b->q8.alloc(size_t(Q) * ix->Db8);
                 b->nq.alloc(Q);
                 GF_HIP(gf::launch_q_i8(b->qf32.p, Q, ix->D, ix->Db8, b->q8.p, b->nq.p, ix->stream));

@@ -307,6 +307,12 @@ struct BfHFinal {
 uint32_t bf_float_dim(int vt, uint32_t D);
 // bf_float_dim, AW 1 or 2, K <= 10.
 bool bf_float_supported(int vt, uint32_t D, uint32_t AW, uint32_t K);
+// Whether records at a padded dimension are made beside an index: they make
+// large exact searches faster and are not needed for any, so they take at most
+// a fifth of the memory that is free once the rows are there.  What the index
+// still needs then fits as it did without them: records are 80 bytes a row at
+// least, a full graph (the largest array to come) 256 at most.
+inline bool bf_pad_records_fit(uint64_t bytes, uint64_t free) { return bytes <= free / 5; }
 // The dimension that the int8 MFMA brute force runs at (D <= 256).
 inline uint32_t bf_i8_dim(uint32_t D) { return (D + 63u) / 64u * 64u; }
 hipError_t launch_bf_float(const BfHArgs& a, int vt, uint32_t AW, uint32_t ncu, hipStream_t st);

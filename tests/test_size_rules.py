@@ -63,3 +63,15 @@ def test_float_items_are_whole_where_many_and_even(rule):
     assert rule("float_item_tiles", 976, 976 * 64, 128, 10_000) == whole
     assert rule("float_item_tiles", 976, 976 * 64, 129, 10_000) == chunk
     assert rule("float_item_tiles", 976, 976 * 64, 96, 64) == chunk
+
+
+@pytest.mark.parametrize("D,dim,elem", [(4, 64, 1), (100, 128, 1), (100, 128, 4), (264, 512, 2), (520, 768, 2)])
+def test_pad_records_leave_room_for_the_index(rule, D, dim, elem):
+    """Records at a padded dimension are made only where a full graph of 64
+    edges a row, the largest array behind them, and its scratch still fit."""
+    N = 1_000_000
+    rec = N // 16 * (dim * 16 * elem + 16 * 4 * 4)   # rows, norms, row ids and attribute words
+    assert rule("pad_records_fit", rec, 5 * rec) == 1
+    assert rule("pad_records_fit", rec, 5 * rec - 1) == 0
+    for free in (rec, rec + 260 * N - 1):
+        assert rule("pad_records_fit", rec, free) == 0 or free - rec >= 260 * N
