@@ -119,6 +119,8 @@ _SYMBOLS = {
                         C.c_uint32, C.c_int32, C.c_void_p, C.c_void_p, C.POINTER(BuildStats)],
     "gf_optimize_graphs": [C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p, C.c_uint32, C.c_uint32, C.c_int32,
                            C.c_void_p, C.POINTER(C.c_double)],
+    "gf_optimize_graphs_in": [C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p, C.c_uint32, C.c_uint32, C.c_int32,
+                              C.c_uint64, C.c_void_p, C.POINTER(C.c_double)],
     "gf_kmeans": [C.c_void_p, C.c_int32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p, C.c_int32,
                   C.c_void_p, C.c_void_p, C.POINTER(C.c_double)],
     "gf_search_noalloc": [C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p, C.POINTER(_NoallocOpts),
@@ -576,15 +578,21 @@ def build_graphs(vectors, global_pid, P, R, E, device=0, graphs=True, cross=True
     return g, x, st
 
 
-def optimize_graphs(knn_graphs, cell_sizes, R, device=0):
+def optimize_graphs(knn_graphs, cell_sizes, R, device=0, max_pairs=None):
     """gf_optimize_graphs: the kNN graphs (N, I) -> optimised graphs (N, R)
-    (rank-based reordering by detourable routes, then reverse edges)."""
+    (rank-based reordering by detourable routes, then reverse edges).
+    max_pairs bounds the second step's scratch (gf_optimize_graphs_in)."""
     g = _c(knn_graphs, np.uint32)
     sz = _c(cell_sizes, np.uint32)
     N, I = g.shape
     out = np.empty((N, R), np.uint32)
     ms = C.c_double()
-    _check(load().gf_optimize_graphs(_ptr(g), N, I, _ptr(sz), sz.size, R, device, _ptr(out), C.byref(ms)))
+    if max_pairs is None:
+        st = load().gf_optimize_graphs(_ptr(g), N, I, _ptr(sz), sz.size, R, device, _ptr(out), C.byref(ms))
+    else:
+        st = load().gf_optimize_graphs_in(_ptr(g), N, I, _ptr(sz), sz.size, R, device, max_pairs, _ptr(out),
+                                          C.byref(ms))
+    _check(st)
     return out, ms.value
 
 

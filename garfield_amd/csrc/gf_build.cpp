@@ -386,7 +386,7 @@ void build_graphs(const void* vectors, int32_t vec_dtype, uint32_t N, uint32_t D
 }
 
 void optimize_graphs(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t* cell_size, uint32_t P,
-                     uint32_t R, int32_t device, uint32_t* graphs, double* ms) {
+                     uint32_t R, int32_t device, uint64_t max_pairs, uint32_t* graphs, double* ms) {
     const auto t0 = std::chrono::steady_clock::now();
     GF_REQUIRE(knn && cell_size && graphs, GF_E_ARG, "null argument");
     GF_REQUIRE(N > 0 && P > 0, GF_E_ARG, "empty graph");
@@ -416,13 +416,12 @@ void optimize_graphs(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t
     dout.alloc(size_t(N) * R);
     GF_HIP(launch_prune(dk.p, N, I, doff.p, P, dord.p, st));
     // Reverse edges and the final rows, whole cells at a time: as many cells
-    // as keep the pairs' scratch within kRevPairs entries (one cell at least).
-    constexpr size_t kRevPairs = size_t(1) << 28;
+    // as keep the pairs' scratch within max_pairs entries (one cell at least).
     std::vector<uint32_t> cut{0};   // first cell of each group
     uint32_t most = 0;
     for (uint32_t c = 1; c <= P; ++c) {
         const size_t rows = offset[c] - offset[cut.back()];
-        if (rows * R > kRevPairs && c - 1 > cut.back()) cut.push_back(c - 1);
+        if (rows * R > max_pairs && c - 1 > cut.back()) cut.push_back(c - 1);
     }
     cut.push_back(P);
     for (size_t g = 0; g + 1 < cut.size(); ++g) most = std::max(most, offset[cut[g + 1]] - offset[cut[g]]);

@@ -1825,7 +1825,13 @@ gf_status gf_build_graphs(const void* vectors, int32_t vec_dtype, uint32_t N, ui
 
 gf_status gf_optimize_graphs(const uint32_t* knn_graphs, uint32_t N, uint32_t I, const uint32_t* cell_size,
                              uint32_t P, uint32_t R, int32_t device, uint32_t* graphs, double* ms) {
-    return run_guarded([&] { gf::optimize_graphs(knn_graphs, N, I, cell_size, P, R, device, graphs, ms); });
+    return run_guarded([&] { gf::optimize_graphs(knn_graphs, N, I, cell_size, P, R, device, gf::kRevPairs, graphs, ms); });
+}
+
+gf_status gf_optimize_graphs_in(const uint32_t* knn_graphs, uint32_t N, uint32_t I, const uint32_t* cell_size,
+                                uint32_t P, uint32_t R, int32_t device, uint64_t max_pairs, uint32_t* graphs,
+                                double* ms) {
+    return run_guarded([&] { gf::optimize_graphs(knn_graphs, N, I, cell_size, P, R, device, max_pairs, graphs, ms); });
 }
 
 gf_status gf_kmeans(const void* vectors, int32_t vec_dtype, uint32_t N, uint32_t D, uint32_t C, uint32_t iters,

@@ -383,6 +383,7 @@ struct RevArgs {
     uint32_t* out;             // N * R
 };
 hipError_t launch_rev_edges(const RevArgs& a, hipStream_t st);
+constexpr uint64_t kRevPairs = uint64_t(1) << 28;   // pairs that a group of cells is held to (2 GiB)
 // k-means update: cnt and fill (C each) must start at zero; start (C) and
 // mem (N) are scratch; centres (C x Dp u8) are rewritten where a cluster
 // has members.

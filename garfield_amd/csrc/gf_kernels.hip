@@ -4490,8 +4490,8 @@ __global__ __launch_bounds__(256) void k_kmeans_mean(const uint8_t* vec, uint32_
     }
 }
 
-// Small id -> value table in LDS (linear probing over 2^k slots, at most
-// half to two thirds full): the slot of `id`, claimed if it is new.
+// Small id -> value table in LDS (linear probing over 2^k slots, at most half
+// full): the slot of `id`, claimed if it is new.
 template <uint32_t SLOTS>
 __device__ __forceinline__ uint32_t id_slot(uint32_t* keys, uint32_t id) {
     uint32_t h = (id * 2654435761u) >> (32 - __builtin_ctz(SLOTS));
@@ -4641,7 +4641,7 @@ __global__ __launch_bounds__(256) void k_rev_fill(RevArgs p) {
 // (rank, node) order, then the rest of the reordered list, each id once; a
 // row still short repeats its first entry.
 __global__ __launch_bounds__(64) void k_rev_merge(RevArgs p) {
-    constexpr uint32_t SLOTS = 256, T = 3;   // at most 32 + 64 + 64 entries
+    constexpr uint32_t SLOTS = 256, T = 2;   // n = I + nrev <= I + R <= 128 entries
     __shared__ uint32_t keys[SLOTS], first[SLOTS];
     __shared__ uint64_t top_[64];
     __shared__ uint32_t seq[64 * T];

@@ -581,7 +581,7 @@ void build_graphs(const void* vectors, int32_t vec_dtype, uint32_t N, uint32_t D
                   uint32_t P, uint32_t R, uint32_t E, int32_t device, uint32_t* cell_graphs, uint32_t* cross,
                   gf_build_stats* stats);
 void optimize_graphs(const uint32_t* knn, uint32_t N, uint32_t I, const uint32_t* cell_size, uint32_t P,
-                     uint32_t R, int32_t device, uint32_t* graphs, double* ms);
+                     uint32_t R, int32_t device, uint64_t max_pairs, uint32_t* graphs, double* ms);
 void kmeans_labels(const void* vectors, int32_t vec_dtype, uint32_t N, uint32_t D, uint32_t C, uint32_t iters,
                    const uint32_t* init_ids, int32_t device, int32_t* labels, uint8_t* centres, double* ms);
 }  // namespace gf

@@ -407,14 +407,20 @@ gf_status gf_build_graphs(const void* vectors, int32_t vec_dtype, uint32_t N, ui
  * concatenated in cell order, cell-local ids, rows ordered by distance, e.g.
  * gf_build_graphs with R = I) is reordered by ascending (number of detourable
  * two-hop routes, rank): the edge at rank k to D has a detour through every
- * B at a rank below k that lists D at a rank below k (GPU).  Then (host) every
- * pruned edge A -> B among the first R adds A to B's reverse list (ranks in
+ * B at a rank below k that lists D at a rank below k.  Then every pruned edge A -> B among the first R adds A to B's reverse list (ranks in
  * order, nodes in order, at most R per list), and the output row keeps the
  * first R/2 reordered edges, then its reverse edges, then the rest of the
  * reordered row, each id once (a row still short repeats its first id).
- * I <= 64, R <= I; ms (wall time of the call) may be NULL. */
+ * I <= 64, R <= I; ms (wall time of the call) may be NULL.  Both steps run on
+ * the GPU, the second in groups of whole cells whose scratch holds 2^28 (node,
+ * rank) pairs of 8 bytes, or one cell's. */
 gf_status gf_optimize_graphs(const uint32_t* knn_graphs, uint32_t N, uint32_t I, const uint32_t* cell_size,
                              uint32_t P, uint32_t R, int32_t device, uint32_t* graphs /*N*R*/, double* ms);
+/* gf_optimize_graphs with the groups' scratch held to max_pairs pairs (one
+ * cell's at least); the same graphs at any value. */
+gf_status gf_optimize_graphs_in(const uint32_t* knn_graphs, uint32_t N, uint32_t I, const uint32_t* cell_size,
+                                uint32_t P, uint32_t R, int32_t device, uint64_t max_pairs,
+                                uint32_t* graphs /*N*R*/, double* ms);
 
 /* Per-point cluster labels for the index (the .cluster file; the reference
  * fits cuVS k-means and predicts, clustering.py:68-87).  Integer Lloyd

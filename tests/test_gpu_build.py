@@ -137,9 +137,9 @@ def test_kmeans_headline_size_property():
     (90, 3, 40, 32, 256),      # cells of about 30 points: rows repeat their nearest
 ])
 def test_optimize_graphs_matches_oracle(N, P, I, R, hi):
-    """gf_optimize_graphs (GPU detour order, host reverse edges and merge) bit
-    for bit against oracle.optimize_graphs, from the library's exact kNN
-    graphs of degree I."""
+    """gf_optimize_graphs (detour order, reverse edges and merge) bit for bit
+    against oracle.optimize_graphs, from the library's exact kNN graphs of
+    degree I."""
     _print_case("optimize", N=N, P=P, I=I, R=R, hi=hi)
     rng = np.random.default_rng(N + I)
     v = rng.integers(0, hi, (N, 64)).astype(np.uint8)
