@@ -1267,7 +1267,7 @@ static void search_resident(gf_batch* b, const gf_search_opts* opts, uint32_t* i
     const uint32_t NS = ix->NS;
     // tiles per item, at most
     const uint32_t tch =
-        gemm_h ? gf::bf_float_item_tiles(NS, ix->ntile, ix->tmax, Q) : gf::bf_item_tiles(NS, Q);
+        gemm_h ? gf::bf_float_item_tiles(fvt == 1, NS, ix->ntile, ix->tmax, Q) : gf::bf_item_tiles(NS, Q);
     b->pass_pending = sched_bf && !b->sel_exact;
     if (sched_bf) {
         if (!b->bcnt.n) {

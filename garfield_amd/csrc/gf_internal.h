@@ -180,19 +180,27 @@ inline uint32_t bf_item_tiles(uint32_t NS, uint32_t Q) {
     return most <= 20000u ? 16u : most <= 65536u ? 32u : kBfMaxItemTiles;
 }
 // The same for the float route, whose items are longer (a workgroup each, a
-// tile record a step): 48, except whole sub-cells where there are many items
-// (NS sub-cells times query groups) and no sub-cell is more than twice the mean
-// (tmax against ntile / NS), so that no long item ends the launch alone.  48 (in
-// even chunks, so 25 to 48) against whole, by the most items there can be, even
-// sub-cells: binary16 7.4k (120k x 768) 807 / 817 us, 13.8k (300k x 96) 520 /
-// 543, 15.4k (250k x 96) 593 / 580, 38k (250k x 768) 1590 / 1530, 153k (1M x
-// 768) 4030 / 3530; fp32 13.8k (300k x 96) 574 / 638, 15.3k (250k x 128) 838 /
-// 835, 31k (500k x 128) 1263 / 1180, 153k (1M x 96) 2830 / 2640.  Sub-cells of
-// skewed attributes, fp32: 300k x 96, 10k queries 2260 / 2950, 1M 5780 / 7260.
-constexpr uint32_t kBfHItemTiles = 48;
-inline uint32_t bf_float_item_tiles(uint32_t NS, uint32_t ntile, uint32_t tmax, uint32_t Q) {
+// tile record a step): 48.  Where there are many items (NS sub-cells times query
+// groups), whole sub-cells if none is more than twice the mean (tmax against
+// ntile / NS), so that no long item ends the launch alone, and 128 for binary16
+// rows if the longest are far beyond that: each of their launches has items
+// enough, and fewer chunks leave fewer keys to re-rank.  48 (in even chunks, so
+// 25 to 48) against whole, by the most items there can be, even sub-cells:
+// binary16 7.4k (120k x 768) 807 / 817 us, 13.8k (300k x 96) 520 / 543, 15.4k
+// (250k x 96) 593 / 580, 38k (250k x 768) 1590 / 1530, 153k (1M x 768) 4030 /
+// 3530; fp32 13.8k (300k x 96) 574 / 638, 15.3k (250k x 128) 838 / 835, 31k (500k
+// x 128) 1263 / 1180, 153k (1M x 96) 2830 / 2640.  Sub-cells of skewed
+// attributes, fp32: 300k x 96, 10k queries 2260 / 2950, 1M 5780 / 7260 (at 128
+// k_bf_f32 alone 5.19 -> 5.46 ms).  Up to 977 tiles (1M x 768 binary16,
+// attributes tied to each other), 48 / 128 / whole: 1000 queries 1050 / 1070 /
+// 1385, 3000 1750 / 1680 / 1700, 10k 4630 / 4360 / 4560; up to 244 (250k) 3000
+// queries 884 / 927 / 1044.
+constexpr uint32_t kBfHItemTiles = 48, kBfHLongItemTiles = 128;
+inline uint32_t bf_float_item_tiles(bool half, uint32_t NS, uint32_t ntile, uint32_t tmax, uint32_t Q) {
     const uint64_t most = uint64_t(NS) * ((Q + 63u) / 64u);
-    return most > 14000u && uint64_t(tmax) * NS <= 2u * uint64_t(ntile) ? kBfMaxItemTiles : kBfHItemTiles;
+    if (most <= 14000u) return kBfHItemTiles;
+    if (uint64_t(tmax) * NS <= 2u * uint64_t(ntile)) return kBfMaxItemTiles;
+    return half && tmax >= 4u * kBfHLongItemTiles ? kBfHLongItemTiles : kBfHItemTiles;
 }
 // Pairs that a batch's lists are first made for, a pair being a (query,
 // sub-cell) combination of one chunk of at most tch tiles: the chunks that n of

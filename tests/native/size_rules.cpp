@@ -12,7 +12,7 @@ int main(int argc, char** argv) {
     if (!std::strcmp(rule, "first_pairs"))
         std::printf("%zu\n", gf::bf_first_pairs(u(2), u(3), u(4), u(5), u(6), u(7)));
     else if (!std::strcmp(rule, "float_item_tiles"))
-        std::printf("%u\n", gf::bf_float_item_tiles(u(2), u(3), u(4), u(5)));
+        std::printf("%u\n", gf::bf_float_item_tiles(u(2) != 0, u(3), u(4), u(5), u(6)));
     else if (!std::strcmp(rule, "pad_records_fit"))
         std::printf("%d\n", int(gf::bf_pad_records_fit(std::strtoull(argv[2], nullptr, 10), std::strtoull(argv[3], nullptr, 10))));
     else

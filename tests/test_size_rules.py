@@ -54,15 +54,20 @@ def test_first_pairs_are_bounded(rule):
     assert rule("first_pairs", 200_000, 64 * 400, 64, 96, 128, 32) == 200_000 * 64
 
 
-def test_float_items_are_whole_where_many_and_even(rule):
+@pytest.mark.parametrize("half", [0, 1])
+def test_float_items_are_whole_where_many_and_even(rule, half):
     """Whole sub-cells from 14001 items up if none is more than twice the
-    mean, chunks of 48 tiles otherwise."""
+    mean, chunks of 128 tiles for binary16 rows if the longest has 512, of 48
+    otherwise."""
     whole, chunk = 65536, 48
-    assert rule("float_item_tiles", 140, 140 * 64, 96, 6400) == chunk
-    assert rule("float_item_tiles", 140, 140 * 64, 96, 6401) == whole
-    assert rule("float_item_tiles", 976, 976 * 64, 128, 10_000) == whole
-    assert rule("float_item_tiles", 976, 976 * 64, 129, 10_000) == chunk
-    assert rule("float_item_tiles", 976, 976 * 64, 96, 64) == chunk
+    assert rule("float_item_tiles", half, 1024, 62500, 511, 10_000) == chunk
+    assert rule("float_item_tiles", half, 1024, 62500, 512, 10_000) == (128 if half else chunk)
+    assert rule("float_item_tiles", half, 100, 62500, 977, 6400) == chunk
+    assert rule("float_item_tiles", half, 140, 140 * 64, 96, 6400) == chunk
+    assert rule("float_item_tiles", half, 140, 140 * 64, 96, 6401) == whole
+    assert rule("float_item_tiles", half, 976, 976 * 64, 128, 10_000) == whole
+    assert rule("float_item_tiles", half, 976, 976 * 64, 129, 10_000) == chunk
+    assert rule("float_item_tiles", half, 976, 976 * 64, 96, 64) == chunk
 
 
 @pytest.mark.parametrize("D,dim,elem", [(4, 64, 1), (100, 128, 1), (100, 128, 4), (264, 512, 2), (520, 768, 2)])
